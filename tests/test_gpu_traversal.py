@@ -1,0 +1,73 @@
+"""Traversal kernels at the edges of their rules: directions outside the quick quotients' range, trees that
+are one leaf, stacks that overflow, queues shorter and longer than one batch per wave."""
+import numpy as np
+import pytest
+
+import yar_amd
+from tests import raygen
+from yar_amd import views as yv
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", ["zero", "two-zero", "tiny", "huge", "denormal", "mixed"])
+def test_directions_outside_the_quick_range(kind, c1_path, oracle):
+    """Zero, denormal, very small and very large direction components take the divided quotients and the
+    case-by-case slab test; hits equal the oracle's bit for bit (the arithmetic is the same)."""
+    scene = yar_amd.Scene(c1_path)
+    rays = raygen.random_rays(scene, 1 << 14, seed=17)
+    d = rays["direction"].astype(np.float64)
+    rng = np.random.default_rng(5)
+    n = rays.size
+    pick = np.zeros((n, 3), bool)
+    pick[np.arange(n), rng.integers(0, 3, n)] = True
+    if kind == "zero":
+        d[pick] = np.where(rng.random(n) < 0.5, 0.0, -0.0)
+    elif kind == "two-zero":
+        d[~pick] = 0.0
+    elif kind == "tiny":
+        d *= 2.0 ** -70
+    elif kind == "huge":
+        d *= 2.0 ** 70
+    elif kind == "denormal":
+        d[pick] = 2.0 ** -140
+    else:
+        d *= 2.0 ** rng.integers(-64, 64, (n, 1)).astype(np.float64)
+        d[pick] *= 2.0 ** -40
+    rays["direction"] = d.astype(np.float32)
+    ctx = yar_amd.Context(scene)
+    for any_hit in (False, True):
+        if any_hit:
+            rays["tmax"] = rng.uniform(0.01, 3.0, n).astype(np.float32)
+        g = ctx.trace_rays(rays, any_hit=any_hit)
+        o = oracle.OracleScene(scene).trace(rays, any_hit=any_hit)
+        assert np.array_equal(g["t"], o["t"], equal_nan=True)
+        if not any_hit:
+            assert np.array_equal(g["object"], o["object"]) and np.array_equal(g["triangle"], o["triangle"])
+
+
+@pytest.mark.parametrize("depth", [1, 4, 16])
+def test_stack_depths_give_the_same_hits(depth, c2_small_path, oracle):
+    scene = yar_amd.Scene(c2_small_path)
+    rays = raygen.random_rays(scene, 1 << 15, seed=23)
+    g = yar_amd.Context(scene, traversal_stack_depth=depth).trace_rays(rays)
+    o = oracle.OracleScene(scene).trace(rays)
+    assert np.array_equal(g["object"], o["object"]) and np.array_equal(g["triangle"], o["triangle"])
+    assert np.array_equal(g["t"], o["t"])
+
+
+@pytest.mark.parametrize("side,grid", [((1, 1), 1), ((7, 3), 3), ((65, 33), 2), ((256, 256), 4), ((640, 416), 2)])
+def test_queue_lengths_and_refill_give_the_same_image(side, grid, c1_path):
+    """A ray's result does not depend on the lanes it shares a wave with: queues of one ray, of less than a
+    batch per wave (spread over all waves) and of several batches, with lanes refilled at 24, 16 and 64
+    idle lanes and in blocks of one and four waves, give the same image bit for bit."""
+    scene = yar_amd.Scene(c1_path)
+    images = []
+    for opts in ({}, {"lane_refill": 1}, {"lane_refill": 2}, {"block_size": 256}, {"max_paths_in_flight": 4096}):
+        ctx = yar_amd.Context(scene, **opts)
+        ctx.set_views([yv.with_film(ctx.view(0), side[0], side[1], grid, seed_offset=3)])
+        img, film, var, st = ctx.render(0)
+        images.append((img, film, var))
+        ctx.close()
+    for img, film, var in images[1:]:
+        assert np.array_equal(img, images[0][0]) and np.array_equal(film, images[0][1]) and var == images[0][2]

@@ -204,7 +204,8 @@ struct yar_gpu_ctx {
     std::vector<yar_view> views;
 
     // scene buffers
-    DevBuf<uint2> scene_nodes, mesh_nodes;
+    DevBuf<uint4> pairs;
+    DevBuf<uint32_t> leaf_ids;
     DevBuf<ObjTrav> objs;
     DevBuf<float4> tri_verts, obj_o2w, obj_nrm, vtx_n;
     DevBuf<int4> obj_info, mesh_info, tri_vidx;
@@ -274,8 +275,7 @@ struct yar_gpu_ctx {
     ~yar_gpu_ctx() {
         if (device >= 0) (void)hipSetDevice(device);
         drop_graph();
-        DevBuf<uint2>* b2[] = {&scene_nodes, &mesh_nodes, &pk};
-        for (auto* b : b2) b->release();
+        pairs.release(); leaf_ids.release(); pk.release();
         objs.release();
         DevBuf<float4>* b4[] = {&tri_verts, &obj_o2w, &obj_nrm, &vtx_n, &ray_o, &ray_d, &coeff, &L, &dl_coeff,
                                 &dl_light, &dl_bsdf, &hit_tb, &radiance, &sh_o, &sh_d, &sh_c, &mi_o, &mi_d,
@@ -307,7 +307,7 @@ struct yar_gpu_ctx {
         lc.scene_stack = info.stack_depth >> 16;
         lc.mesh_stack = info.stack_depth & 0xffff;
         lc.priv_stack = opt.stack_mode == 2;
-        lc.refill = opt.lane_refill == 1;
+        lc.refill = opt.lane_refill == 1 ? 16 : opt.lane_refill == 2 ? 64 : 24;
         lc.counters = opt.enable_counters != 0;
         lc.trav_grid = lc.shadow_grid = lc.mis_grid = 1;
         lc.path_grid = 1;
@@ -362,6 +362,58 @@ static float pbrt3_remap(float r, const yar_render_config& cfg, bool is_alpha) {
     return r * r;
 }
 
+// Device form of a kd-tree (words in the reference's KdNode encoding): how many node pairs (one per
+// interior node) and leaf ids (of leaves with two or more primitives) it takes.
+static void tree_size(const std::vector<uint32_t>& w, int64_t& n_pairs, int64_t& n_ids) {
+    n_pairs = n_ids = 0;
+    for (size_t j = 0; j < w.size() / 2;) {
+        const uint32_t w0 = w[2 * j], count = w0 >> 2;
+        if ((w0 & 3u) != 3u) { n_pairs++; j++; continue; }
+        if (count > 1) n_ids += count;
+        j += 1 + (count > 1 ? count / 2 : 0);
+    }
+}
+
+// Writes a tree's pairs from pair_base on and its leaf ids (plus id_add) from id_base on; returns its root
+// node.  The pairs of three successive levels (up to seven pairs, 112 bytes) lie together, the subtrees
+// behind them depth-first, so a descent touches about one 128-byte line per three levels.
+static uint2 pack_tree(const std::vector<uint32_t>& w, uint32_t pair_base, uint32_t id_base, uint32_t id_add, uint32_t* pairs,
+                       uint32_t* ids) {
+    struct Item { uint32_t node; uint32_t* at; };        // a node and where its two device words go
+    uint2 root = make_uint2(0u, 0u);
+    uint32_t root_words[2] = {0u, 0u}, next_pair = pair_base, next_id = id_base;
+    std::vector<Item> todo{{0u, root_words}}, cluster;
+    while (!todo.empty()) {
+        cluster.assign(1, todo.back());
+        todo.pop_back();
+        const size_t behind = todo.size();
+        size_t level_end = 1;
+        for (size_t k = 0, level = 0; k < cluster.size(); k++) {
+            if (k == level_end) { level++; level_end = cluster.size(); }
+            const Item it = cluster[k];
+            const uint32_t w0 = w[2 * (size_t)it.node], w1 = w[2 * (size_t)it.node + 1];
+            if ((w0 & 3u) == 3u) {
+                const uint32_t count = w0 >> 2;
+                it.at[0] = kNodeLeaf | count;
+                it.at[1] = count == 0 ? 0u : count == 1 ? w1 + id_add : next_id;
+                for (uint32_t j = 0; count > 1 && j < count; j++) ids[next_id++] = w[2 * (size_t)it.node + 1 + j] + id_add;
+            } else if (level == 3) {
+                todo.push_back(it);
+            } else {
+                const uint32_t pair = next_pair++;
+                it.at[0] = (w0 & 3u) << 30 | pair;
+                it.at[1] = w1;
+                cluster.push_back({it.node + 1, pairs + 4 * (size_t)pair});
+                cluster.push_back({w0 >> 2, pairs + 4 * (size_t)pair + 2});
+            }
+        }
+        std::reverse(todo.begin() + behind, todo.end());
+    }
+    root.x = root_words[0];
+    root.y = root_words[1];
+    return root;
+}
+
 static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
     using namespace yar;
     auto t0 = std::chrono::steady_clock::now();
@@ -388,20 +440,32 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
     auto t1 = std::chrono::steady_clock::now();
 
     // flatten meshes
-    std::vector<int64_t> mtri(d->mesh_count + 1, 0), mvtx(d->mesh_count + 1, 0), mnode(d->mesh_count + 1, 0);
+    std::vector<int64_t> mtri(d->mesh_count + 1, 0), mvtx(d->mesh_count + 1, 0);
+    int64_t n_nodes = (int64_t)(stree.words.size() / 2);
     for (int i = 0; i < d->mesh_count; i++) {
         mtri[i + 1] = mtri[i] + d->meshes[i].triangle_count;
         mvtx[i + 1] = mvtx[i] + d->meshes[i].vertex_count;
-        mnode[i + 1] = mnode[i] + (int64_t)(trees[i].words.size() / 2);
+        n_nodes += (int64_t)(trees[i].words.size() / 2);
     }
-    if (mnode[d->mesh_count] >= (int64_t)0x40000000 || mtri[d->mesh_count] >= (int64_t)0x7fffffff)
+    // device trees, the scene tree first: node pairs and leaf ids of each tree in its own range
+    const size_t n_trees = (size_t)d->mesh_count + 1;
+    auto words_of = [&](size_t t) -> const std::vector<uint32_t>& { return t == 0 ? stree.words : trees[t - 1].words; };
+    std::vector<int64_t> pair_base(n_trees + 1, 0), id_base(n_trees + 1, 0);
+    parallel_for(n_trees, [&](size_t t) { tree_size(words_of(t), pair_base[t + 1], id_base[t + 1]); }, 1);
+    for (size_t t = 0; t < n_trees; t++) { pair_base[t + 1] += pair_base[t]; id_base[t + 1] += id_base[t]; }
+    if (n_nodes >= (int64_t)0x40000000 || id_base[n_trees] > (int64_t)0xffffffff || mtri[d->mesh_count] >= (int64_t)0x7fffffff)
         throw HipError{"scene exceeds 2^30 kd nodes or 2^31 triangles", YAR_ERR_CAPACITY};
+    std::vector<uint4> kp((size_t)pair_base[n_trees]);
+    std::vector<uint32_t> kids((size_t)id_base[n_trees]);
+    std::vector<uint2> roots(n_trees);
+    parallel_for(n_trees, [&](size_t t) {
+        roots[t] = pack_tree(words_of(t), (uint32_t)pair_base[t], (uint32_t)id_base[t], t == 0 ? 0u : (uint32_t)mtri[t - 1], reinterpret_cast<uint32_t*>(kp.data()), kids.data());
+    }, 1);
     std::vector<float4> tv(3 * (size_t)mtri[d->mesh_count]);
     std::vector<int4> tvi(mtri[d->mesh_count]);
     std::vector<float4> vn(std::max<int64_t>(1, mvtx[d->mesh_count]), make_float4(0, 0, 0, 0));
     std::vector<float2> vuv(std::max<int64_t>(1, mvtx[d->mesh_count]), make_float2(0, 0));
     std::vector<int4> minfo(d->mesh_count);
-    std::vector<uint2> mn(std::max<int64_t>(1, mnode[d->mesh_count]));
     int mesh_depth = 0;
     for (int i = 0; i < d->mesh_count; i++) {
         const yar_mesh_desc& m = d->meshes[i];
@@ -421,29 +485,8 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
             if (m.uvs) vuv[mvtx[i] + v] = make_float2(m.uvs[2 * v], m.uvs[2 * v + 1]);
         }
         minfo[i] = make_int4(mflags, 0, 0, 0);
-        // rebase the mesh tree: above_child and leaf triangle ids become global indices
-        const std::vector<uint32_t>& w = trees[i].words;
-        size_t nn = w.size() / 2;
-        uint32_t nb = (uint32_t)mnode[i], tb = (uint32_t)mtri[i];
-        size_t j = 0;
-        while (j < nn) {
-            uint32_t w0 = w[2 * j], w1 = w[2 * j + 1];
-            if ((w0 & 3u) != 3u) {
-                mn[nb + j] = make_uint2((w0 & 3u) | (((w0 >> 2) + nb) << 2), w1);
-                j++;
-            } else {
-                uint32_t cnt = w0 >> 2;
-                size_t span = 1 + (cnt > 1 ? cnt / 2 : 0);
-                std::vector<uint32_t> ws(w.begin() + 2 * j, w.begin() + 2 * (j + span));
-                for (uint32_t q = 0; q < cnt; q++) ws[1 + q] += tb;
-                for (size_t q = 0; q < span; q++) mn[nb + j + q] = make_uint2(ws[2 * q], ws[2 * q + 1]);
-                j += span;
-            }
-        }
         mesh_depth = std::max(mesh_depth, trees[i].depth);
     }
-    std::vector<uint2> sn(stree.words.size() / 2);
-    for (size_t j = 0; j < sn.size(); j++) sn[j] = make_uint2(stree.words[2 * j], stree.words[2 * j + 1]);
 
     // objects
     std::vector<ObjTrav> ot(d->object_count);
@@ -455,20 +498,21 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
         const KdBuildResult& t = trees[o.mesh];
         ObjTrav& r = ot[i];
         m34_rows(o.world_to_object, r.w2o0, r.w2o1, r.w2o2);
-        uint32_t root = (uint32_t)mnode[o.mesh], tb = (uint32_t)mtri[o.mesh];
-        float rootf, tbf;
-        std::memcpy(&rootf, &root, 4);
-        std::memcpy(&tbf, &tb, 4);
-        r.lo_node = make_float4(t.bounds.lo.x, t.bounds.lo.y, t.bounds.lo.z, rootf);
-        r.hi_tri = make_float4(t.bounds.hi.x, t.bounds.hi.y, t.bounds.hi.z, tbf);
+        const uint2 root = roots[(size_t)o.mesh + 1];
+        const int tb = (int)mtri[o.mesh];
+        float root_x, root_y;
+        std::memcpy(&root_x, &root.x, 4);
+        std::memcpy(&root_y, &root.y, 4);
+        r.lo_root = make_float4(t.bounds.lo.x, t.bounds.lo.y, t.bounds.lo.z, root_x);
+        r.hi_root = make_float4(t.bounds.hi.x, t.bounds.hi.y, t.bounds.hi.z, root_y);
         m34_rows(o.object_to_world, o2w[3 * i], o2w[3 * i + 1], o2w[3 * i + 2]);
         // object_to_world_normal_transform = transpose of world_to_object's 3x3 (scene_loader.cpp:56-62)
         const float* w2o = o.world_to_object;
         nrm[3 * i] = make_float4(w2o[0], w2o[4], w2o[8], 0.f);
         nrm[3 * i + 1] = make_float4(w2o[1], w2o[5], w2o[9], 0.f);
         nrm[3 * i + 2] = make_float4(w2o[2], w2o[6], w2o[10], 0.f);
-        oinfo[i] = make_int4(o.material, o.area_light, o.mesh, (int)tb);
-        ctx->tri_base[i] = (int32_t)tb;
+        oinfo[i] = make_int4(o.material, o.area_light, o.mesh, tb);
+        ctx->tri_base[i] = tb;
     }
     std::vector<DevMaterial> mats(std::max(1, d->material_count));
     bool has_mix = false;
@@ -645,8 +689,8 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
     }
 
     hipStream_t s = ctx->stream;
-    ctx->scene_nodes.upload(sn, s);
-    ctx->mesh_nodes.upload(mn, s);
+    ctx->pairs.upload(kp, s);
+    ctx->leaf_ids.upload(kids, s);
     ctx->objs.upload(ot, s);
     ctx->tri_verts.upload(tv, s);
     ctx->tri_vidx.upload(tvi, s);
@@ -669,8 +713,9 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
     auto t2 = std::chrono::steady_clock::now();
 
     DevScene& S = ctx->scene;
-    S.scene_nodes = ctx->scene_nodes.p;
-    S.mesh_nodes = ctx->mesh_nodes.p;
+    S.pairs = ctx->pairs.p;
+    S.leaf_ids = ctx->leaf_ids.p;
+    S.root = roots[0];
     S.objs = ctx->objs.p;
     S.tri_verts = ctx->tri_verts.p;
     S.scene_lo = make_float4(stree.bounds.lo.x, stree.bounds.lo.y, stree.bounds.lo.z, 0.f);
@@ -703,7 +748,7 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
                  d->sphere_light_count + d->mesh_light_count + d->environment_light_count;                            // update_total_light_count, light.cpp:35
 
     yar_gpu_info& inf = ctx->info;
-    inf.scene_bytes = (int64_t)(sn.size() * 8 + mn.size() * 8 + ot.size() * sizeof(ObjTrav) + tv.size() * 16 +
+    inf.scene_bytes = (int64_t)(kp.size() * sizeof(uint4) + kids.size() * 4 + ot.size() * sizeof(ObjTrav) + tv.size() * 16 +
                                 tvi.size() * 16 + vn.size() * 16 + vuv.size() * 8 + o2w.size() * 32 + oinfo.size() * 16);
     inf.triangle_count = mtri[d->mesh_count];
     inf.object_count = d->object_count;
@@ -712,8 +757,7 @@ static void upload_scene(yar_gpu_ctx* ctx, const yar_scene_desc* d) {
     int req = ctx->opt.traversal_stack_depth;
     int sd, md;
     // Default: 8-entry short stacks per level (restart beyond).  Deeper LDS stacks cost occupancy
-    // (a 32-entry stack pair is 64 KB per 128-thread block) and measured 2x slower on both the
-    // 2M-triangle and the 2k-triangle scenes, with bit-identical results.
+    // (a 32-entry stack pair is 32 KB per wave) with bit-identical results.
     if (req <= 0) req = 8;
     sd = std::min(pow2_at_least(req), pow2_at_least(std::max(1, stree.depth)));
     md = std::min(pow2_at_least(req), pow2_at_least(std::max(1, mesh_depth)));

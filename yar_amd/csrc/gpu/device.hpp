@@ -37,6 +37,10 @@ YG_INLINE V3 cross(V3 a, V3 b) { return v3(a.y * b.z - a.z * b.y, a.z * b.x - a.
 YG_INLINE float len_sq(V3 a) { return a.x * a.x + a.y * a.y + a.z * a.z; }
 YG_INLINE float length(V3 a) { return sqrtf(len_sq(a)); }
 YG_INLINE V3 normalized(V3 a) { return vdiv(a, length(a)); }
+// Component a of (x, y, z), from values: selecting between members of a struct in memory would be
+// turned into an indexed load and keep the struct there.
+YG_INLINE float pick(float x, float y, float z, uint32_t a) { return a == 0u ? x : (a == 1u ? y : z); }
+YG_INLINE float pick(float x, float y, float z, bool is_x, bool is_xy) { return is_x ? x : (is_xy ? y : z); }
 YG_INLINE V3 from4(float4 f) { return v3(f.x, f.y, f.z); }
 
 // ColorRGB semantics: division by a scalar multiplies by its reciprocal (src/lib/color.h:104).
@@ -70,9 +74,16 @@ YG_INLINE V3 xform_vector(const M34& m, V3 v) {
 }
 
 // ---- scene layout in HBM ---------------------------------------------------------------
-// Object record for traversal (80 bytes): world_to_object rows, mesh-tree bounds with the
-// mesh's root node index and triangle base packed into the w lanes.
-struct ObjTrav { float4 w2o0, w2o1, w2o2, lo_node, hi_tri; };
+// kd node: 8 bytes, the two children of an interior node side by side in one 16-byte pair, so a
+// traversal requests both as soon as it knows the parent and picks one when its decision is made (the
+// load no longer waits for the decision's arithmetic, nor the decision for the load).
+// x: axis (0, 1, 2) << 30 | pair of the children, y: split position; leaf: x = 3 << 30 | count, y = the
+// primitive of a one-primitive leaf, else the leaf's first entry in the leaf id array.
+constexpr uint32_t kNodeY = 1u << 30, kNodeZ = 2u << 30, kNodeLeaf = 3u << 30, kNodeIndex = (1u << 30) - 1u;
+
+// Object record for traversal (80 bytes): world_to_object rows, mesh-tree bounds with the root node of
+// the mesh tree in the w lanes.
+struct ObjTrav { float4 w2o0, w2o1, w2o2, lo_root, hi_root; };
 
 // Device-only material codes: rough glass (yar_material_desc type GLASS with roughness > 0), the
 // pbrt3 uber material and the mix material.
@@ -102,8 +113,10 @@ struct DevSphere { float4 p; float4 L; };
 struct DevEnv { float4 l2w0, l2w1, l2w2, w2l0, w2l1, w2l2, L; };
 
 struct DevScene {
-    const uint2* scene_nodes;
-    const uint2* mesh_nodes;       // all mesh trees; interior above_child and leaf ids rebased
+    // node pairs of the scene tree and all mesh trees; leaf ids are object indices / global triangles
+    const uint4* pairs;
+    const uint32_t* leaf_ids;
+    uint2 root;                    // root node of the scene tree
     const ObjTrav* objs;
     const float4* tri_verts;       // 3 float4 per triangle (object space)
     float4 scene_lo, scene_hi;
@@ -130,38 +143,73 @@ struct DevScene {
     int has_mix;                   // some material is a mix
 };
 
+// ---- correctly rounded quotients without the compiler's scaled division ------------------
+// Newton step on the hardware reciprocal with the residual taken by a fused multiply-add (Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor", 1990): the result is
+// the correctly rounded 1/x for every x whose magnitude lies in [2^-126, 2^126].
+constexpr float kRcpMin = 0x1p-126f, kRcpMax = 0x1p126f;
+YG_INLINE float rcp_rn(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
+}
+// Correctly rounded a / b from r = rcp_rn(b): two residual corrections of a * r (the first makes the
+// quotient faithful, the second rounds it, as above).  For 2^-60 <= |a| <= |b| <= 2^60.
+YG_INLINE float div_rn(float a, float b, float r) {
+    const float q = a * r;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q1, a), r, q1);
+}
+// Directions whose components all lie here take the quick quotients and the branch-free slab test.
+YG_INLINE bool quick_direction(V3 d) {
+    const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
+    return fminf(fminf(ax, ay), az) >= 0x1p-60f && fmaxf(fmaxf(ax, ay), az) <= 0x1p60f;
+}
+
 // ---- ray/box slab test (Bounding_Box::intersect_by_ray_without_NaNs, bounding_box.h:63) ----
-YG_INLINE bool slab(float4 lo, float4 hi, V3 o, V3 d, float& tmin, float& tmax) {
-    float t0 = 0.f, t1 = f_inf();
-    float los[3] = {lo.x, lo.y, lo.z}, his[3] = {hi.x, hi.y, hi.z};
-    float os[3] = {o.x, o.y, o.z}, ds[3] = {d.x, d.y, d.z};
+// inv receives 1 / d.  For a quick direction the two plane distances of an axis are ordered by min and
+// max, and since t0 only grows and t1 only shrinks one comparison at the end decides; other directions
+// (zero components among them) follow the reference's cases.
+YG_INLINE bool slab(float4 lo, float4 hi, V3 o, V3 d, bool quick, V3& inv, float& tmin, float& tmax) {
+    V3 r = v3(rcp_rn(d.x), rcp_rn(d.y), rcp_rn(d.z));
+    const float ax = (lo.x - o.x) * r.x, bx = (hi.x - o.x) * r.x;
+    const float ay = (lo.y - o.y) * r.y, by = (hi.y - o.y) * r.y;
+    const float az = (lo.z - o.z) * r.z, bz = (hi.z - o.z) * r.z;
+    float t0 = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fmaxf(fminf(az, bz), 0.f));
+    float t1 = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fminf(fmaxf(az, bz), f_inf()));
+    bool outside = false;
+    if (!quick) {
+        r = v3(1.f / d.x, 1.f / d.y, 1.f / d.z);
+        t0 = 0.f;
+        t1 = f_inf();
+        const float los[3] = {lo.x, lo.y, lo.z}, his[3] = {hi.x, hi.y, hi.z};
+        const float os[3] = {o.x, o.y, o.z}, ds[3] = {d.x, d.y, d.z}, is[3] = {r.x, r.y, r.z};
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        if (ds[i] != 0.f) {
-            float inv = 1.f / ds[i];
-            float s0 = (los[i] - os[i]) * inv;
-            float s1 = (his[i] - os[i]) * inv;
-            if (inv < 0.f) { float t = s0; s0 = s1; s1 = t; }
-            t0 = s0 > t0 ? s0 : t0;
-            t1 = s1 < t1 ? s1 : t1;
-            if (t0 > t1) return false;
-        } else if (os[i] < los[i] || os[i] > his[i]) {
-            return false;
+        for (int i = 0; i < 3; i++) {
+            if (ds[i] != 0.f) {
+                float s0 = (los[i] - os[i]) * is[i];
+                float s1 = (his[i] - os[i]) * is[i];
+                if (is[i] < 0.f) { const float t = s0; s0 = s1; s1 = t; }
+                t0 = s0 > t0 ? s0 : t0;
+                t1 = s1 < t1 ? s1 : t1;
+            } else {
+                outside = outside || os[i] < los[i] || os[i] > his[i];
+            }
         }
     }
+    inv = r;
     tmin = t0; tmax = t1;
-    return true;
+    return !(t0 > t1) && !outside;
 }
 
 // ---- watertight ray/triangle test (intersection.cpp:53-113) ------------------------------
-YG_INLINE float watertight(V3 o, V3 d, int kx, int ky, int kz, float sx, float sy, float sz,
-                           float4 p0, float4 p1, float4 p2, V3& b) {
-    V3 a0 = v3(p0.x - o.x, p0.y - o.y, p0.z - o.z);
-    V3 a1 = v3(p1.x - o.x, p1.y - o.y, p1.z - o.z);
-    V3 a2 = v3(p2.x - o.x, p2.y - o.y, p2.z - o.z);
-    float p0x = a0[kx], p0y = a0[ky], p0z = a0[kz];
-    float p1x = a1[kx], p1y = a1[ky], p1z = a1[kz];
-    float p2x = a2[kx], p2y = a2[ky], p2z = a2[kz];
+YG_INLINE float watertight(V3 o, uint32_t kz, float sx, float sy, float sz, float4 p0, float4 p1, float4 p2, V3& b) {
+    const V3 a0 = v3(p0.x - o.x, p0.y - o.y, p0.z - o.z);
+    const V3 a1 = v3(p1.x - o.x, p1.y - o.y, p1.z - o.z);
+    const V3 a2 = v3(p2.x - o.x, p2.y - o.y, p2.z - o.z);
+    // the permutations are the rotations (kx, ky, kz) = (1, 2, 0), (2, 0, 1), (0, 1, 2)
+    const float p0x = pick(a0.y, a0.z, a0.x, kz), p0y = pick(a0.z, a0.x, a0.y, kz), p0z = pick(a0.x, a0.y, a0.z, kz);
+    const float p1x = pick(a1.y, a1.z, a1.x, kz), p1y = pick(a1.z, a1.x, a1.y, kz), p1z = pick(a1.x, a1.y, a1.z, kz);
+    const float p2x = pick(a2.y, a2.z, a2.x, kz), p2y = pick(a2.z, a2.x, a2.y, kz), p2z = pick(a2.x, a2.y, a2.z, kz);
     float x0 = p0x + sx * p0z, y0 = p0y + sy * p0z;
     float x1 = p1x + sx * p1z, y1 = p1y + sy * p1z;
     float x2 = p2x + sx * p2z, y2 = p2y + sy * p2z;
@@ -179,7 +227,8 @@ YG_INLINE float watertight(V3 o, V3 d, int kx, int ky, int kz, float sx, float s
     float z0 = sz * p0z, z1 = sz * p1z, z2 = sz * p2z;
     float ts = e0 * z0 + e1 * z1 + e2 * z2;
     if ((fbits(det) ^ fbits(ts)) >> 31) return f_inf();
-    float inv_det = 1.f / det;
+    float inv_det = rcp_rn(det);
+    if (!(fabsf(det) >= kRcpMin && fabsf(det) <= kRcpMax)) inv_det = 1.f / det;
     float t = inv_det * ts;
     b = v3(e0 * inv_det, e1 * inv_det, e2 * inv_det);
     return t;
@@ -195,267 +244,266 @@ struct TravCounters { uint32_t nodes, leaf_refs, tri_tests, objects; };
 
 struct HitRec { float t; int obj; uint32_t tri; V3 b; };
 
-// Short traversal stack in LDS: entries [slot][lane] so a wave's accesses hit distinct banks.
-// When a push finds the stack full the oldest entry is dropped; when the stack then runs empty
-// the traversal restarts from the root at the current exit distance (kd-restart), visiting the
-// remaining leaves in the same front-to-back order.  With depth >= tree depth it is the plain
-// stack traversal of kdtree.cpp:219-439.
+// Short traversal stacks of both tree levels in LDS, one 8-byte entry (child, exit distance) per slot and
+// lane, laid out [slot][lane] per wave; slots [0, depth) belong to the scene tree, [depth, 2 depth) to
+// the mesh tree being visited.  When a push finds a level's stack full its oldest entry is dropped; when
+// the stack then runs empty the traversal restarts from the level's root at the current exit distance
+// (kd-restart), visiting the remaining leaves in the same front-to-back order.  With depth >= tree depth
+// it is the plain stack traversal of kdtree.cpp:219-439.
+// Depth 8 keeps five waves per SIMD resident (8 KB of LDS per wave).  Entries that hold the child's node
+// words save the load of a pop, but at 12 bytes either leave 13 waves per CU (1024x1024 frame of the
+// 2.2M-triangle scene: 95 ms against 84) or four entries per level, whose restarts cost the small frames
+// 7% (637x359 at 4 spp: 8.6 ms against 8.05); one ring shared by both levels restarts the scene level and
+// is worse than either (9.9 ms).
+constexpr int kStackEntryBytes = 8;
 struct LdsStack {
-    uint32_t* node;
-    float* tmax;
-    int stride;
-    YG_INLINE void put(int slot, uint32_t n, float t) { node[slot * stride] = n; tmax[slot * stride] = t; }
-    YG_INLINE void get(int slot, uint32_t& n, float& t) const { n = node[slot * stride]; t = tmax[slot * stride]; }
+    uint2* e;
+    YG_INLINE void put(uint32_t slot, uint32_t n, float t) { e[slot << 6] = make_uint2(n, fbits(t)); }
+    YG_INLINE uint2 get(uint32_t slot) const { return e[slot << 6]; }
 };
 
 // The same stack in per-lane private memory (scratch): no LDS footprint, so occupancy is bounded by
 // registers only; accesses are lane-interleaved by the hardware and stay in the vector L1.
 template <int N>
 struct PrivStack {
-    uint32_t node[N];
-    float tmax[N];
-    YG_INLINE void put(int slot, uint32_t n, float t) { node[slot] = n; tmax[slot] = t; }
-    YG_INLINE void get(int slot, uint32_t& n, float& t) const { n = node[slot]; t = tmax[slot]; }
+    uint2 e[N];
+    YG_INLINE void put(uint32_t slot, uint32_t n, float t) { e[slot] = make_uint2(n, fbits(t)); }
+    YG_INLINE uint2 get(uint32_t slot) const { return e[slot]; }
 };
-
-// Leaf id j of a leaf whose first id is in word1 of node `nd` (kdtree.h:53: ids packed inline).
-YG_INLINE uint32_t leaf_id(const uint2* __restrict__ nodes, uint32_t nd, uint32_t first, uint32_t j) {
-    if (j == 0) return first;
-    uint2 w = nodes[nd + ((j + 1) >> 1)];
-    return (j & 1) ? w.x : w.y;
-}
-
-// Short-stack bookkeeping of one tree level packed in one word: push pointer in bits 0-7 (used
-// modulo the stack size, a power of two dividing 256), live entries in bits 8-15, bit 16 set
-// when entries were dropped since the last restart, bit 17 set while a descent is suspended.
-constexpr uint32_t kSsCount = 1u << 8, kSsDropped = 1u << 16, kSsResume = 1u << 17;
-
-// Interior nodes a lane descends per traversal step (a constant, so the descent is unrolled).
-constexpr int kDescentBudget = 6;
-YG_INLINE uint32_t ss_count(uint32_t ss) { return (ss >> 8) & 0xffu; }
-YG_INLINE uint32_t ss_push(uint32_t ss) { return (ss & ~0xffu) | ((ss + 1u) & 0xffu); }
-YG_INLINE uint32_t ss_pop(uint32_t ss) { return ((ss & ~0xffu) | ((ss - 1u) & 0xffu)) - kSsCount; }
-
-// One step of a kd-tree descent shared by both levels: interior node -> child (pushing the far
-// child when the ray straddles the split), as KdTree::intersect's inner loop (kdtree.cpp:245-290).
-template <class Stack>
-YG_INLINE void kd_interior(uint2 w, uint32_t& node, V3 o, V3 d, V3 inv, float& tmin, float& tmax, Stack& st,
-                           int mask, int depth, uint32_t& ss) {
-    // Written as selects so a wave runs one straight-line sequence whatever mix of cases its lanes
-    // are in; only the stack write is a branch.
-    const uint32_t axis = w.x & 3u;
-    const float oa = axis == 0u ? o.x : (axis == 1u ? o.y : o.z);
-    const float da = axis == 0u ? d.x : (axis == 1u ? d.y : d.z);
-    const float ia = axis == 0u ? inv.x : (axis == 1u ? inv.y : inv.z);
-    const float dist = bitsf(w.y) - oa;
-    const uint32_t below = node + 1, above = w.x >> 2;
-    const bool pos = dist > 0.f;
-    const uint32_t first = pos ? below : above;
-    const uint32_t second = pos ? above : below;
-    const float ts = dist * ia;
-    const bool zero = dist == 0.f;
-    const bool only_first = ts > tmax || ts < 0.f;
-    const bool only_second = !only_first && ts < tmin;
-    const bool push = !zero && !only_first && !only_second;
-    const uint32_t next = only_second ? second : first;
-    const uint32_t on_plane = da > 0.f ? above : below;
-    if (push) st.put((int)(ss & (uint32_t)mask), second, tmax);
-    const uint32_t pushed = ss_push(ss);
-    const uint32_t ss_new = ss_count(ss) == (uint32_t)depth ? (pushed | kSsDropped) : (pushed + kSsCount);
-    ss = push ? ss_new : ss;
-    tmax = push ? ts : tmax;
-    node = zero ? on_plane : next;
-}
-
-// After a leaf: pop the next subtree, or restart behind the last leaf when the short stack dropped
-// entries (kd-restart; a restart that would not advance steps past the degenerate point), or finish.
-// Returns false when the level's traversal is complete.
-template <class Stack>
-YG_INLINE bool kd_next(uint32_t& node, uint32_t root, float& tmin, float& tmax, float t1, Stack& st, int mask, uint32_t& ss,
-                       float& restart_t) {
-    if (ss_count(ss) > 0) {
-        ss = ss_pop(ss);
-        uint32_t nn; float tm;
-        st.get((int)(ss & (uint32_t)mask), nn, tm);
-        node = nn;
-        tmin = tmax;
-        tmax = tm;
-        return true;
-    }
-    if ((ss & kSsDropped) && tmax < t1) {
-        ss &= ~kSsDropped;
-        node = root;
-        tmin = tmax > restart_t ? tmax : nextafterf(restart_t, f_inf());
-        restart_t = tmin;
-        tmax = t1;
-        return true;
-    }
-    return false;
-}
 
 // Two-level closest-hit / any-hit query over the scene tree and the per-mesh trees
 // (KdTree::intersect / intersect_any with intersect_scene_geometry_data and
-// intersect_triangle_mesh_geometry_data, kdtree.cpp:12-109), as a resumable per-lane state
-// machine.  Both levels run in one loop: each step() advances a lane by one node of whichever tree
-// it is in (scene tree, or the mesh tree of the object being visited), so lanes inside a mesh tree
-// and lanes still descending the scene tree make progress together, and a persistent kernel can
-// hand a lane a new ray as soon as its query ends.  The visit order and hit updates are those of
-// the nested traversal, so results are identical.
+// intersect_triangle_mesh_geometry_data, kdtree.cpp:12-109), as a per-lane state machine whose
+// actions a wave takes by vote.  A lane is at one of four places: on its way down a tree (scene or
+// mesh: the same code, on the ray of that level), behind a finished leaf, at an object of a scene
+// leaf, or at a triangle of a mesh leaf.  The order of a lane's own actions is that of the nested
+// traversal, so its hit is identical whatever the other lanes of its wave do.
+// What bounds it is instruction issue under divergence: every vector instruction is issued for the whole
+// wave, and with each lane taking its own next action the lanes did useful work in 19% of the issue slots
+// (closest hit, 1024x1024 frame of the 2.2M-triangle scene; 71 ms per frame).  Waiting for company per
+// action, one descent code for both levels and lanes that take new rays while others finish theirs
+// (trace_queue) bring that to 43 ms, child pairs requested before the decision to 39 ms.
+// Cap on a wave's turns, which only guarantees that every wave terminates; real trees need far fewer.
+constexpr uint32_t kMaxTurns = 1u << 28;
+
 template <bool ANY, bool COUNT>
 struct Tracer {
-    V3 o, d, inv;
-    float any_t, tmax_in, st1;
-    HitRec hit;
-    bool found_any;
-    // scene level
-    uint32_t snode;
-    float stmin, stmax, srestart;
-    uint32_t sss;                   // packed short-stack state
-    // objects of the current scene leaf still to visit
-    uint32_t lnode, lfirst, ln, lj;
-    // mesh level
-    bool in_mesh;
-    uint32_t mroot, mnode, oi;
-    float mtmin, mtmax, mt1, mrestart;
-    uint32_t mss;                   // packed short-stack state
-    V3 lo, ld, linv;
-    uint32_t kxyz;                  // watertight axis permutation kx | ky << 2 | kz << 4
+    enum : uint32_t { kDone = 0, kObject = 1, kTriangle = 2, kDescend = 3, kLeafDone = 4 };
+    // Interior nodes a lane descends per turn (a constant, so the steps are unrolled): 2, 3, 4 and 6 took
+    // 85, 83.9, 83.5 and 87 ms on the 1024x1024 frame of the 2.2M-triangle scene.
+    static constexpr int kDescents = 4;
+    V3 o, d, inv;                   // world ray
+    float tmax_in;
+    HitRec hit;                     // hit.t bounds the query (any hit: stays at tmax)
+    uint32_t phase;
+    bool in_mesh, found_any;
+    // current level: ray origin and reciprocal direction, node words, ray interval, its exit, restart point
+    // and the stack's top and bottom (entries are numbered as pushed; those from bottom on are live)
+    V3 co, ci;
+    uint32_t node_x, node_y;
+    float tmin, tmax, t1, restart_t;
+    int top, bottom;
+    uint32_t item, item_at, item_end;       // objects or triangles of the current leaf still to visit
+    // scene level while a mesh is visited
+    float s_tmax, s_t1, s_restart;
+    int s_top, s_bottom;
+    uint32_t s_item, s_at, s_end;
+    uint32_t oi;
+    uint32_t kz;                    // watertight set-up (intersection.cpp:55-61)
     float sx, sy, sz;
-    int iter;
 
-    // Returns false when the ray misses the scene bounds (the query is then already complete).
-    YG_INLINE bool start(const DevScene& s, V3 o_, V3 d_, float tmax_) {
-        o = o_; d = d_; tmax_in = tmax_; any_t = tmax_;
+    // A ray that misses the scene bounds is complete at once (phase kDone).
+    YG_INLINE void start(const DevScene& s, V3 o_, V3 d_, float tmax_) {
+        o = o_; d = d_; tmax_in = tmax_;
         hit.t = tmax_; hit.obj = -1; hit.tri = 0; hit.b = v3(0, 0, 0);
         found_any = false;
-        float t0, t1;
-        if (!slab(s.scene_lo, s.scene_hi, o, d, t0, t1)) return false;
-        inv = v3(1.f / d.x, 1.f / d.y, 1.f / d.z);
-        st1 = t1;
-        snode = 0; stmin = t0; stmax = t1; srestart = -1.f; sss = 0u;
-        lnode = lfirst = ln = lj = 0;
+        const bool inside = slab(s.scene_lo, s.scene_hi, o, d, quick_direction(d), inv, tmin, tmax);
+        t1 = tmax;
+        node_x = s.root.x; node_y = s.root.y; restart_t = -1.f; top = bottom = 0;
+        co = o; ci = inv;
         in_mesh = false;
-        iter = 0;
-        return true;
+        phase = inside && hit.t > tmin ? kDescend : kDone;
     }
 
     // closest hit: hit.t < tmax_in; any hit: found_any
     YG_INLINE bool result() const { return ANY ? found_any : hit.t < tmax_in; }
 
-    // One traversal step; returns true when the query is complete.  A lane outside a mesh tree
-    // takes the scene-level actions in traversal order, each at most once per step: finish the
-    // current scene leaf, descend to the next one, set up its next object; a lane inside a mesh
-    // tree (possibly just entered) then processes one mesh leaf.  A descent stops after
-    // kDescentBudget interior nodes and resumes from the same node in the next step, so a lane far
-    // from its next leaf does not hold the wave while the other lanes wait at theirs.
-    template <class SStack, class MStack>
-    YG_INLINE bool step(const DevScene& s, SStack& sst, int sdepth, MStack& mst, int mdepth, TravCounters& cnt) {
-        // The iteration cap only guarantees that every wave terminates; real trees need far fewer.
-        if (++iter > (1 << 24)) return true;
-        if (!in_mesh) {
-            if (ln > 0 && lj >= ln) {
-                // the leaf's objects are done: continue the scene traversal behind it
-                ln = 0;
-                if (!kd_next(snode, 0u, stmin, stmax, st1, sst, sdepth - 1, sss, srestart)) return true;
+    // One interior node on the way down: to a child, pushing the far one when the ray straddles the
+    // split, as KdTree::intersect's inner loop (kdtree.cpp:245-290).  Both children are requested before
+    // the decision, and a pushed node keeps its words, so neither waits for memory on its own.  Written
+    // as selects so a wave runs one straight-line sequence whatever mix of cases its lanes are in.
+    template <class Stack>
+    YG_INLINE void descend(const DevScene& s, Stack& st, int depth, TravCounters& cnt) {
+        const uint4 p = s.pairs[node_x & kNodeIndex];
+        if (COUNT) cnt.nodes++;
+        const bool is_x = node_x < kNodeY, is_xy = node_x < kNodeZ;
+        const float oa = pick(co.x, co.y, co.z, is_x, is_xy), ia = pick(ci.x, ci.y, ci.z, is_x, is_xy);
+        const float dist = bitsf(node_y) - oa;
+        const float ts = dist * ia;
+        const bool pos = dist > 0.f, on_plane = dist == 0.f;
+        const bool only_first = ts > tmax || ts < 0.f || on_plane;
+        const bool only_second = !only_first && ts < tmin;
+        const bool push = !only_first && !only_second;
+        bool below = pos != only_second;                 // the child to go to
+        if (on_plane) {
+            // the origin lies on the plane: the side the ray leaves to
+            V3 cd = d;
+            if (in_mesh) {
+                const ObjTrav ob = s.objs[oi];
+                cd = xform_vector(M34{ob.w2o0, ob.w2o1, ob.w2o2}, d);
             }
-            if (ln == 0) {
-                if (!((ANY ? any_t : hit.t) > stmin)) return true;
-                if (COUNT && !(sss & kSsResume)) cnt.nodes++;
-                sss &= ~kSsResume;
-                uint2 w = s.scene_nodes[snode];
-                for (int b = kDescentBudget; (w.x & 3u) != 3u;) {
-                    if (b-- == 0) {
-                        sss |= kSsResume;
-                        return false;
-                    }
-                    kd_interior(w, snode, o, d, inv, stmin, stmax, sst, sdepth - 1, sdepth, sss);
-                    if (COUNT) cnt.nodes++;
-                    w = s.scene_nodes[snode];
-                }
-                const uint32_t n = w.x >> 2;
-                if (COUNT) cnt.leaf_refs += n;
-                if (n == 0) return !kd_next(snode, 0u, stmin, stmax, st1, sst, sdepth - 1, sss, srestart);
-                lnode = snode; lfirst = w.y; ln = n; lj = 0;
-            }
-            // next object of the scene leaf: ray to object space, mesh bounds, watertight setup
-            oi = leaf_id(s.scene_nodes, lnode, lfirst, lj);
-            lj++;
-            const ObjTrav ob = s.objs[oi];
-            if (COUNT) cnt.objects++;
-            const M34 w2o = {ob.w2o0, ob.w2o1, ob.w2o2};
-            lo = xform_point(w2o, o);
-            ld = xform_vector(w2o, d);
-            float mt0;
-            if (!slab(ob.lo_node, ob.hi_tri, lo, ld, mt0, mt1)) return false;
-            linv = v3(1.f / ld.x, 1.f / ld.y, 1.f / ld.z);
-            mroot = fbits(ob.lo_node.w);
-            // watertight-test setup hoisted per mesh ray (intersection.cpp:55-61)
-            const float ax = fabsf(ld.x), ay = fabsf(ld.y), az = fabsf(ld.z);
-            const int kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
-            const int kx = (kz == 2 ? 0 : kz + 1);
-            const int ky = (kz == 0 ? 2 : kz - 1);
-            kxyz = (uint32_t)kx | ((uint32_t)ky << 2) | ((uint32_t)kz << 4);
-            const float dx = ld[kx], dy = ld[ky], dz = ld[kz];
-            sx = -dx / dz; sy = -dy / dz; sz = linv[kz];           // linv[kz] is 1.f / dz
-            mnode = mroot; mtmin = mt0; mtmax = mt1; mrestart = -1.f;
-            mss = 0u;
-            in_mesh = true;
+            below = !(pick(cd.x, cd.y, cd.z, is_x, is_xy) > 0.f);
         }
-        // one leaf of the current mesh tree
-        bool done = !((ANY ? any_t : hit.t) > mtmin);
-        if (!done) {
-            // descend to the next leaf: neither the loop bound nor tmin changes on the way down
-            if (COUNT && !(mss & kSsResume)) cnt.nodes++;
-            mss &= ~kSsResume;
-            uint2 w = s.mesh_nodes[mnode];
-            for (int b = kDescentBudget; (w.x & 3u) != 3u;) {
-                if (b-- == 0) {
-                    mss |= kSsResume;
-                    return false;
-                }
-                kd_interior(w, mnode, lo, ld, linv, mtmin, mtmax, mst, mdepth - 1, mdepth, mss);
-                if (COUNT) cnt.nodes++;
-                w = s.mesh_nodes[mnode];
+        if (push) {
+            st.put((in_mesh ? (uint32_t)depth : 0u) + ((uint32_t)top & (uint32_t)(depth - 1)), (node_x & kNodeIndex) << 1 | (below ? 1u : 0u), tmax);
+            top++;
+            bottom = max(bottom, top - depth);
+            tmax = ts;
+        }
+        node_x = below ? p.x : p.z;
+        node_y = below ? p.y : p.w;
+    }
+
+    // A leaf: to its first object or triangle.
+    YG_INLINE void leaf(const DevScene& s, TravCounters& cnt) {
+        const uint32_t n = node_x & kNodeIndex;
+        if (COUNT) { cnt.nodes++; cnt.leaf_refs += n; }
+        item = node_y;
+        item_at = node_y;
+        item_end = node_y + n;
+        if (n > 1u) item = s.leaf_ids[node_y];
+        phase = n == 0u ? kLeafDone : in_mesh ? kTriangle : kObject;
+    }
+
+    // Behind a leaf: the level's next subtree from the stack, or a restart behind the leaf when the
+    // short stack dropped entries (a restart that would not advance steps past the degenerate point).
+    // A finished mesh returns to the scene leaf's next object, or behind that leaf.
+    template <class Stack>
+    YG_INLINE void leaf_done(const DevScene& s, Stack& st, int depth) {
+        bool more = top > bottom;
+        if (more) {
+            top--;
+            tmin = tmax;
+            const uint2 e = st.get((in_mesh ? (uint32_t)depth : 0u) + ((uint32_t)top & (uint32_t)(depth - 1)));
+            const uint2 n = reinterpret_cast<const uint2*>(s.pairs)[e.x];
+            node_x = n.x; node_y = n.y;
+            tmax = bitsf(e.y);
+        }
+        if (!more && bottom > 0 && tmax < t1) {
+            top = bottom = 0;
+            node_x = s.root.x; node_y = s.root.y;
+            if (in_mesh) { node_x = fbits(s.objs[oi].lo_root.w); node_y = fbits(s.objs[oi].hi_root.w); }
+            tmin = tmax > restart_t ? tmax : nextafterf(restart_t, f_inf());
+            restart_t = tmin;
+            tmax = t1;
+            more = true;
+        }
+        more = more && hit.t > tmin;
+        phase = more ? kDescend : kDone;
+        if (!more && in_mesh) {
+            co = o; ci = inv;
+            tmax = s_tmax; t1 = s_t1; restart_t = s_restart; top = s_top; bottom = s_bottom;
+            item = s_item; item_at = s_at; item_end = s_end;
+            phase = item_at < item_end ? kObject : kLeafDone;
+        }
+        in_mesh = in_mesh && more;
+    }
+
+    // Next object of the scene leaf: ray to object space, mesh bounds, watertight set-up.
+    YG_INLINE void object(const DevScene& s, TravCounters& cnt) {
+        oi = item;
+        const ObjTrav ob = s.objs[oi];
+        item_at++;
+        if (item_at < item_end) item = s.leaf_ids[item_at];
+        if (COUNT) cnt.objects++;
+        const M34 w2o = {ob.w2o0, ob.w2o1, ob.w2o2};
+        const V3 lo = xform_point(w2o, o);
+        const V3 ld = xform_vector(w2o, d);
+        const bool quick = quick_direction(ld);
+        V3 li;
+        float m0, m1;
+        const bool inside = slab(ob.lo_root, ob.hi_root, lo, ld, quick, li, m0, m1);
+        phase = item_at < item_end ? kObject : kLeafDone;
+        if (inside && hit.t > m0) {
+            s_tmax = tmax; s_t1 = t1; s_restart = restart_t; s_top = top; s_bottom = bottom;
+            s_item = item; s_at = item_at; s_end = item_end;
+            co = lo; ci = li;
+            const float ax = fabsf(ld.x), ay = fabsf(ld.y), az = fabsf(ld.z);
+            kz = (ax > ay) ? (ax > az ? 0u : 2u) : (ay > az ? 1u : 2u);
+            const float dz = pick(ld.x, ld.y, ld.z, kz);
+            const float dx = pick(ld.y, ld.z, ld.x, kz);
+            const float dy = pick(ld.z, ld.x, ld.y, kz);
+            sz = pick(li.x, li.y, li.z, kz);
+            sx = div_rn(-dx, dz, sz);
+            sy = div_rn(-dy, dz, sz);
+            if (!quick) {
+                sx = -dx / dz;
+                sy = -dy / dz;
             }
-            const uint32_t n = w.x >> 2;
-            if (COUNT) cnt.leaf_refs += n;
-            for (uint32_t k = 0; k < n; k++) {
-                const uint32_t ti = leaf_id(s.mesh_nodes, mnode, w.y, k);
-                const float4 p0 = s.tri_verts[3 * (size_t)ti], p1 = s.tri_verts[3 * (size_t)ti + 1],
-                             p2 = s.tri_verts[3 * (size_t)ti + 2];
-                if (COUNT) cnt.tri_tests++;
-                V3 b;
-                const float t = watertight(lo, ld, (int)(kxyz & 3u), (int)((kxyz >> 2) & 3u), (int)(kxyz >> 4), sx, sy,
-                                           sz, p0, p1, p2, b);
+            node_x = fbits(ob.lo_root.w); node_y = fbits(ob.hi_root.w);
+            tmin = m0; tmax = m1; t1 = m1; restart_t = -1.f; top = bottom = 0;
+            in_mesh = true;
+            phase = kDescend;
+        }
+    }
+
+    // Next triangle of the mesh leaf.
+    YG_INLINE void triangle(const DevScene& s, TravCounters& cnt) {
+        const uint32_t ti = item;
+        const float4 p0 = s.tri_verts[3 * (size_t)ti], p1 = s.tri_verts[3 * (size_t)ti + 1], p2 = s.tri_verts[3 * (size_t)ti + 2];
+        item_at++;
+        if (item_at < item_end) item = s.leaf_ids[item_at];
+        phase = item_at < item_end ? kTriangle : kLeafDone;
+        if (COUNT) cnt.tri_tests++;
+        V3 b;
+        const float t = watertight(co, kz, sx, sy, sz, p0, p1, p2, b);
+        if (ANY ? !(t >= hit.t) : t < hit.t) {
+            if (!degenerate(p0, p1, p2)) {
                 if (ANY) {
-                    if (t >= any_t) continue;
-                    if (degenerate(p0, p1, p2)) continue;
                     found_any = true;
-                    return true;
-                } else if (t < hit.t) {
-                    if (degenerate(p0, p1, p2)) continue;
+                    phase = kDone;
+                } else {
                     hit.t = t; hit.tri = ti; hit.b = b; hit.obj = (int)oi;
                 }
             }
-            done = !kd_next(mnode, mroot, mtmin, mtmax, mt1, mst, mdepth - 1, mss, mrestart);
         }
-        if (done) {
-            in_mesh = false;
-        }
-        return false;
     }
+
+    // One turn of the wave's calling lanes.  Objects and triangles wait until at least as many lanes
+    // want them as go down the trees, so each action runs with many lanes rather than in every lane's
+    // turn order.
+    template <class Stack>
+    YG_INLINE void turn(const DevScene& s, Stack& st, int depth, TravCounters& cnt) {
+        if (phase == kLeafDone) leaf_done(s, st, depth);
+#pragma unroll
+        for (int k = 0; k < kDescents; k++)
+            if (phase == kDescend && node_x < kNodeLeaf) descend(s, st, depth, cnt);
+        if (phase == kDescend && node_x >= kNodeLeaf) leaf(s, cnt);
+        const int n_down = wave_count(phase >= kDescend);
+        const int n_tri = wave_count(phase == kTriangle);
+        if (n_tri > 0 && n_tri >= n_down)
+            if (phase == kTriangle) triangle(s, cnt);
+        const int n_obj = wave_count(phase == kObject);
+        if (n_obj > 0 && n_obj >= n_down)
+            if (phase == kObject) object(s, cnt);
+    }
+    // Calling lanes for which p holds, as a scalar.
+    YG_INLINE static int wave_count(bool p) { return __builtin_amdgcn_readfirstlane((int)__popcll(__ballot(p))); }
 };
 
-// Runs one query to completion.
-template <bool ANY, bool COUNT, class SStack, class MStack>
-YG_INLINE bool trace(const DevScene& s, V3 o, V3 d, float tmax_in, HitRec& hit, SStack& sst, int sdepth,
-                     MStack& mst, int mdepth, TravCounters& cnt) {
+// Runs one query per calling lane to completion.
+template <bool ANY, bool COUNT, class Stack>
+YG_INLINE bool trace(const DevScene& s, V3 o, V3 d, float tmax_in, HitRec& hit, Stack& st, int depth, TravCounters& cnt) {
     Tracer<ANY, COUNT> tr;
-    if (tr.start(s, o, d, tmax_in))
-        while (!tr.step(s, sst, sdepth, mst, mdepth, cnt)) {}
+    tr.start(s, o, d, tmax_in);
+    for (uint32_t turn = 0; turn < kMaxTurns; turn++) {
+        if (__ballot(tr.phase != tr.kDone) == 0ull) break;
+        tr.turn(s, st, depth, cnt);
+    }
     hit = tr.hit;
     return tr.result();
 }
+
 
 // ---- PCG32 (third-party/pcg/pcg_basic.c:46-75) ------------------------------------------
 constexpr uint64_t kPcgMult = 6364136223846793005ULL;

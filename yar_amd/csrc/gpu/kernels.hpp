@@ -128,7 +128,7 @@ struct LaunchCfg {
     int block;                // threads per block for traversal kernels
     int scene_stack, mesh_stack;
     bool priv_stack;          // stacks in private (scratch) memory instead of LDS
-    bool refill;              // per-lane refill in the persistent traversal kernels
+    int refill;               // idle lanes at which a wave of a persistent traversal kernel takes new rays
     bool counters;
     int trav_grid;            // persistent traversal grids (blocks): k_extend, k_shadow, k_mis
     int shadow_grid, mis_grid;

@@ -12,6 +12,7 @@
 // sampling are the only libm calls on the path).
 #include "kernels.hpp"
 #include "shading.hpp"
+#include <algorithm>
 
 namespace yg {
 
@@ -546,108 +547,80 @@ void launch_raygen(const Chunk* c, long long n_paths_max, const Paths& p, Queues
 // BSDF-sampled light rays, direct_lighting.cpp:163-191).  Persistent: each wave fetches 64 rays
 // at a time from a device cursor until the queue is drained.
 // ---------------------------------------------------------------------------------------------
-struct StackCfg { int sd, md, refill; };
-
-YG_INLINE void lds_stacks(uint32_t* lds_base, StackCfg sc, LdsStack& sst, LdsStack& mst) {
-    const int T = blockDim.x, t = threadIdx.x;
-    uint32_t* snode = lds_base;
-    float* stm = reinterpret_cast<float*>(lds_base + sc.sd * T);
-    uint32_t* mnode = lds_base + 2 * sc.sd * T;
-    float* mtm = reinterpret_cast<float*>(lds_base + 2 * sc.sd * T + sc.md * T);
-    sst = LdsStack{snode + t, stm + t, T};
-    mst = LdsStack{mnode + t, mtm + t, T};
-}
+struct StackCfg { int depth, refill; };
 
 constexpr int kPrivDepth = 32;   // private stack capacity per level (restart beyond)
 
-// Runs `body(sst, sd, mst, md)` with the stacks of the selected storage.
+// Runs `body(stack, depth)` with the stacks of the selected storage.
 template <bool PRIV, class Body>
 YG_INLINE void with_stacks(StackCfg cfg, Body body) {
     if (PRIV) {
-        PrivStack<kPrivDepth> sst, mst;
-        body(sst, min(cfg.sd, kPrivDepth), mst, min(cfg.md, kPrivDepth));
+        PrivStack<2 * kPrivDepth> st;
+        body(st, min(cfg.depth, kPrivDepth));
     } else {
-        extern __shared__ uint32_t lds_u[];
-        LdsStack sst, mst;
-        lds_stacks(lds_u, cfg, sst, mst);
-        body(sst, cfg.sd, mst, cfg.md);
+        extern __shared__ uint2 lds_stack[];
+        LdsStack st{lds_stack + (threadIdx.x >> 6) * (uint32_t)(128 * cfg.depth) + (threadIdx.x & 63u)};
+        body(st, cfg.depth);
     }
 }
 
-// Persistent traversal over a device queue.  With `refill` a lane whose query ended takes the next
-// queue entry as soon as at least 16 lanes of its wave are idle, so a wave is not held by its
-// longest ray (pays on small scenes with short, uneven queries); otherwise waves take batches of 64.
+// Persistent traversal over a device queue.  A wave takes runs of `size` entries: the first one is its by
+// position (no atomic, so a launch over a short queue costs almost nothing), the others come from the
+// cursor, 256 entries at a time while more than 8 fetches per wave remain (fewer same-address atomics),
+// then 64 (balanced tail).  A lane whose query ended takes the run's next entry once cfg.refill lanes of
+// its wave are idle, so a wave is not held by its longest ray (24 idle lanes against 64, i.e. whole
+// batches: 84 against 103 ms on the 1024x1024 frame of the 2.2M-triangle scene, 8 and 32 within 1%).
+// A queue of less than a batch per wave is spread over all waves: one ray's chain of dependent loads and
+// branches is what such a launch lasts, and in a wave of its own a ray does not wait for 63 others
+// (64x64 tile at 4 spp: 2.7 to 1.7 ms per render).
 // setup(index, o, d, tmax) returns the payload finish(payload, tracer) receives.
-template <bool ANY, bool COUNT, class SStack, class MStack, class Setup, class Finish>
-YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, SStack& sst, int sd, MStack& mst, int md,
-                           TravCounters& cnt, bool refill, Setup setup, Finish finish) {
+template <bool ANY, bool COUNT, class Stack, class Setup, class Finish>
+YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Stack& st, int depth, TravCounters& cnt,
+                           StackCfg cfg, Setup setup, Finish finish) {
     Tracer<ANY, COUNT> tr;
-    if (!refill) {
-        // batches of 64: every lane of the wave runs its query to completion before the next batch.
-        // The first `size` entries of every wave are assigned statically (no atomic, so a launch
-        // over a short queue costs almost nothing); further work comes from the cursor, 4 batches
-        // per update while more than 8 fetches per wave remain (fewer same-address atomics), then
-        // single batches (balanced tail).
-        const uint32_t wpb = (blockDim.x + 63u) >> 6;
-        const uint32_t waves = gridDim.x * wpb;
-        uint32_t size = n > 8u * 256u * waves ? 256u : 64u;
-        const uint32_t static_end = waves * size;
-        for (uint32_t base = (blockIdx.x * wpb + (threadIdx.x >> 6)) * size; base < n;
-             base = static_end + wave_fetch(cursor, size)) {
-            const uint32_t end = min(base + size, n);
-            for (uint32_t b = base; b < end; b += 64u) {
-                const uint32_t i = b + __lane_id();
-                if (i < end) {
-                    V3 o, d;
-                    float tmax;
-                    const uint32_t payload = setup(i, o, d, tmax);
-                    if (tr.start(sc, o, d, tmax))
-                        while (!tr.step(sc, sst, sd, mst, md, cnt)) {}
-                    finish(payload, tr);
-                }
-            }
-            if (n - end < 8u * 256u * waves) size = 64u;
-        }
-        return;
-    }
-    bool busy = false, exhausted = false;
-    uint32_t payload = 0;
+    tr.phase = tr.kDone;
+    const uint32_t wpb = (blockDim.x + 63u) >> 6;
+    const uint32_t waves = gridDim.x * wpb;
+    uint32_t size = n > 8u * 256u * waves ? 256u : 64u;
+    if (n < 64u * waves) size = max(1u, (n + waves - 1u) / waves);
+    const uint32_t static_end = waves * size;
     const uint32_t lane = __lane_id();
-    for (;;) {
-        const uint64_t idle = __ballot(!busy);
-        const uint32_t n_idle = (uint32_t)__popcll(idle);
-        if (!exhausted && (n_idle >= 16 || n_idle == 64)) {
-            const int leader = __ffsll((unsigned long long)idle) - 1;
-            uint32_t base = 0;
-            if ((int)lane == leader) base = atomicAdd(cursor, n_idle);
-            base = __shfl(base, leader);
-            exhausted = base + n_idle >= n;
-            if (!busy) {
-                const uint32_t idx = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                if (idx < n) {
+    uint32_t next = __builtin_amdgcn_readfirstlane((blockIdx.x * wpb + (threadIdx.x >> 6)) * size);
+    uint32_t end = min(next + size, n);
+    bool more = static_end < n;
+    bool has = false;
+    uint32_t payload = 0;
+    for (uint32_t turn = 0; turn < kMaxTurns; turn++) {
+        const uint64_t idle = __ballot(tr.phase == tr.kDone);
+        const int n_idle = __builtin_amdgcn_readfirstlane((int)__popcll(idle));
+        if (n_idle >= cfg.refill) {
+            if (tr.phase == tr.kDone && has) { finish(payload, tr); has = false; }
+            if (next >= end && more) {
+                next = __builtin_amdgcn_readfirstlane(static_end + wave_fetch(cursor, size));
+                end = min(next + size, n);
+                more = next < n;
+                if (size == 256u && n - min(end, n) < 8u * 256u * waves) size = 64u;
+            }
+            if (next < end) {
+                const uint32_t i = next + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                if (tr.phase == tr.kDone && i < end) {
                     V3 o, d;
                     float tmax;
-                    payload = setup(idx, o, d, tmax);
-                    busy = tr.start(sc, o, d, tmax);
-                    if (!busy) finish(payload, tr);                  // missed the scene bounds
+                    payload = setup(i, o, d, tmax);
+                    tr.start(sc, o, d, tmax);
+                    has = true;
                 }
+                next = min(next + (uint32_t)n_idle, end);
+            } else if (n_idle == 64) {
+                break;
             }
         }
-        if (__ballot(busy) == 0) {
-            if (exhausted) break;
-            continue;
-        }
-        if (busy && tr.step(sc, sst, sd, mst, md, cnt)) {
-            finish(payload, tr);
-            busy = false;
-        }
+        tr.turn(sc, st, depth, cnt);
     }
 }
 
-// The closest-hit and shadow traversals are latency bound: registers capped for five waves per SIMD
-// (96 VGPRs; four waves at the uncapped 105) measured faster on config 2 (k_shadow 28.4 -> 27.0 ms
-// per step with no spills, k_extend 74.9 -> 74.3 ms with 28-36 B of spills); k_mis keeps its registers
-// (40 B of spills there cost more than the wave gains).  Blocks of at most 256 threads.
+// Registers capped for the five waves per SIMD that the stacks' LDS allows (80 to 90 VGPRs, no spills; a
+// sixth wave needs 80, spills 28 B in k_extend and gains nothing).  Blocks of at most 256 threads.
 #define YG_TRAV_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 
 template <bool COUNT, bool PRIV>
@@ -659,8 +632,8 @@ __global__ void YG_TRAV_BOUNDS k_extend(DevScene sc, Paths P, Queues q, int pari
         atomicAdd(&q.totals[19], 1ull);
     }
     TravCounters cnt = {0, 0, 0, 0};
-    with_stacks<PRIV>(cfg, [&](auto& sst, int sd, auto& mst, int md) {
-        trace_queue<false, COUNT>(sc, n, &q.counts[6], sst, sd, mst, md, cnt, cfg.refill != 0,
+    with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
+        trace_queue<false, COUNT>(sc, n, &q.counts[6], st, depth, cnt, cfg,
             [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
                 const uint32_t slot = in[i];
                 o = from4(P.ray_o[slot]);
@@ -682,8 +655,8 @@ __global__ void YG_TRAV_BOUNDS k_shadow(DevScene sc, Paths P, Queues q, StackCfg
     const uint32_t n = q.counts[2];
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&q.totals[17], (unsigned long long)n);
     TravCounters cnt = {0, 0, 0, 0};
-    with_stacks<PRIV>(cfg, [&](auto& sst, int sd, auto& mst, int md) {
-        trace_queue<true, COUNT>(sc, n, &q.counts[7], sst, sd, mst, md, cnt, cfg.refill != 0,
+    with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
+        trace_queue<true, COUNT>(sc, n, &q.counts[7], st, depth, cnt, cfg,
             [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
                 const float4 o4 = q.shadow_o[i];
                 o = from4(o4);
@@ -699,12 +672,12 @@ __global__ void YG_TRAV_BOUNDS k_shadow(DevScene sc, Paths P, Queues q, StackCfg
 }
 
 template <bool COUNT, bool PRIV>
-__global__ void __launch_bounds__(256) k_mis(DevScene sc, Paths P, Queues q, StackCfg cfg) {
+__global__ void YG_TRAV_BOUNDS k_mis(DevScene sc, Paths P, Queues q, StackCfg cfg) {
     const uint32_t n = q.counts[3];
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&q.totals[18], (unsigned long long)n);
     TravCounters cnt = {0, 0, 0, 0};
-    with_stacks<PRIV>(cfg, [&](auto& sst, int sd, auto& mst, int md) {
-        trace_queue<false, COUNT>(sc, n, &q.counts[8], sst, sd, mst, md, cnt, cfg.refill != 0,
+    with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
+        trace_queue<false, COUNT>(sc, n, &q.counts[8], st, depth, cnt, cfg,
             [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
                 o = from4(q.mis_o[i]);
                 d = from4(q.mis_d[i]);
@@ -1535,12 +1508,12 @@ __global__ __launch_bounds__(256) void k_bin_local(Paths P, Queues q, int parity
 
 static size_t stack_lds(const LaunchCfg& cfg) {
     if (cfg.priv_stack) return 0;
-    return (size_t)2 * (cfg.scene_stack + cfg.mesh_stack) * cfg.block * sizeof(uint32_t);
+    return (size_t)2 * std::max(cfg.scene_stack, cfg.mesh_stack) * cfg.block * kStackEntryBytes;
 }
 
 #define YG_LAUNCH_TRAV(KERNEL, GRID, ...)                                                                  \
     do {                                                                                                   \
-        StackCfg st{cfg.scene_stack, cfg.mesh_stack, cfg.refill ? 1 : 0};                                  \
+        StackCfg st{std::max(cfg.scene_stack, cfg.mesh_stack), cfg.refill};                               \
         dim3 grid_((unsigned)(GRID)), block_(cfg.block);                                                   \
         size_t shm = stack_lds(cfg);                                                                       \
         if (cfg.counters) {                                                                                \
@@ -1785,15 +1758,15 @@ __global__ void k_trace_rays(DevScene sc, const float4* __restrict__ rays, long 
     if (i < n) {
         const float4 o4 = rays[2 * i], d4 = rays[2 * i + 1];
         HitRec h;
-        with_stacks<PRIV>(cfg, [&](auto& sst, int sd, auto& mst, int md) {
+        with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
             if (any) {
-                bool occ = trace<true, COUNT>(sc, from4(o4), from4(d4), o4.w, h, sst, sd, mst, md, cnt);
+                bool occ = trace<true, COUNT>(sc, from4(o4), from4(d4), o4.w, h, st, depth, cnt);
                 out_tb[i] = make_float4(occ ? 1.f : 0.f, 0.f, 0.f, 0.f);
                 out_ot[i] = make_int2(-1, -1);
             } else {
-                bool found = trace<false, COUNT>(sc, from4(o4), from4(d4), o4.w, h, sst, sd, mst, md, cnt);
+                bool found = trace<false, COUNT>(sc, from4(o4), from4(d4), o4.w, h, st, depth, cnt);
                 if (found) {
-                    const int tri_base = fbits(sc.objs[h.obj].hi_tri.w);
+                    const int tri_base = sc.obj_info[h.obj].w;
                     out_tb[i] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
                     out_ot[i] = make_int2(h.obj, (int)h.tri - tri_base);
                 } else {
