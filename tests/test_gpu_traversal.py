@@ -71,3 +71,28 @@ def test_queue_lengths_and_refill_give_the_same_image(side, grid, c1_path):
         ctx.close()
     for img, film, var in images[1:]:
         assert np.array_equal(img, images[0][0]) and np.array_equal(film, images[0][1]) and var == images[0][2]
+
+
+@pytest.mark.parametrize("opts", [{}, {"use_graph": 1}, {"bin_rays": 2}, {"enable_timing": 1}], ids=["eager", "graph", "binned", "timed"])
+@pytest.mark.parametrize("depth,grid,region", [(11, (1, 1), (0, 0, 33, 17)), (12, (3, 3), (100, 60, 171, 131)), (24, (4, 5), (90, 90, 140, 113))])
+def test_deep_paths_in_flight_match_one_sample_per_pass(depth, grid, region, opts, scene_dir):
+    """Beyond ten bounces: all samples in flight with the pixel's parked samples resumed in order, against
+    one sample per pixel per pass (paths in flight below one tile's samples), bit for bit and ray for ray."""
+    path = yar_amd.generate_scene(1, str(scene_dir / f"c1_depth{depth}.pbrt"), seed=1)
+    text = open(path).read()
+    # a white room keeps more paths alive past the tables
+    lines = [l if not l.startswith('Material "matte"') else 'Material "matte" "rgb Kd" [ 0.95 0.95 0.95 ]' for l in text.splitlines()]
+    text = "\n".join(lines).replace('"integer maxdepth" [ 5 ]', f'"integer maxdepth" [ {depth} ]') + "\n"
+    open(path, "w").write(text)
+    scene = yar_amd.Scene(path)
+    out = []
+    for o in (opts, {"max_paths_in_flight": 16}):
+        ctx = yar_amd.Context(scene, **o)
+        ctx.set_views([yv.with_film(ctx.view(0), 256, 256, grid, seed_offset=5, region=region)])
+        for _ in range(2):
+            img, film, var, st = ctx.render(0)
+            out.append((img, film, var, st.closest_rays, st.any_rays))
+        ctx.close()
+    for img, film, var, closest, any_rays in out[1:]:
+        assert np.array_equal(img, out[0][0]) and np.array_equal(film, out[0][1]) and var == out[0][2]
+        assert (closest, any_rays) == (out[0][3], out[0][4])

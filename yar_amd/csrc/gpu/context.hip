@@ -235,6 +235,7 @@ struct yar_gpu_ctx {
     DevBuf<uint2> pk;
     DevBuf<uint32_t> state;
     DevBuf<uint64_t> rng;
+    DevBuf<int> first_parked;
     DevBuf<uint32_t> q_a, q_b, sh_path, mi_path, dl_path, counts, q_unsorted;
     DevBuf<float4> sh_o, sh_d, sh_c, mi_o, mi_d, mi_f;
     DevBuf<float> mi_ndw;
@@ -283,7 +284,7 @@ struct yar_gpu_ctx {
         for (auto* b : b4) b->release();
         DevBuf<int4>* bi4[] = {&obj_info, &mesh_info, &tri_vidx, &side_info};
         for (auto* b : bi4) b->release();
-        DevBuf<int>* bi[] = {&pix_view, &tile_first, &side_view};
+        DevBuf<int>* bi[] = {&pix_view, &tile_first, &side_view, &first_parked};
         for (auto* b : bi) b->release();
         vtx_uv.release(); materials.release(); rects.release(); points.release();
         spots.release(); dirs.release(); mesh_lights.release(); mesh_light_cdf.release(); spheres.release(); env.release();
@@ -313,6 +314,7 @@ struct yar_gpu_ctx {
         lc.path_grid = 1;
         lc.stream = stream;
         lc.guided = false;
+        lc.fallback = false;
         lc.net = GuideNet{nullptr, nullptr, nullptr};
         lc.guide_grid = 0;
         return lc;
@@ -895,7 +897,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     const int n_dims = d1 + d2;                                               // shuffled sampler runs per pixel
     // RNG fallback past 10 bounces couples a pixel's samples; guided passes draw those dimensions
     // from each path's own stream instead
-    const bool sequential = rc.max_light_bounces > 10 && !guided;
+    const bool fallback = rc.max_light_bounces > 10 && !guided;
 
     // views, tile offsets and the pixel list
     std::vector<DevView> dv;
@@ -945,6 +947,12 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b > 0)
             max_paths = std::max<int64_t>((int64_t)1 << 16, std::min<int64_t>(max_paths, (int64_t)(free_b / 4) / per_path));
     }
+    // Paths past ten bounces: all samples in flight, those that reach the fallback stream resumed in sample
+    // order behind them (depth-16 crop of 19,200 pixels at 64 spp: 368 ms with one sample per pixel per
+    // pass, 33 ms so), unless one tile's samples already exceed the paths in flight.
+    int64_t tile_paths = 0;
+    for (const Unit& u : units) tile_paths = std::max(tile_paths, u.count * dv[u.part].spp);
+    const bool sequential = fallback && tile_paths > max_paths, deep = fallback && !sequential;
     const int perm_bytes = job_max_spp <= 256 ? 1 : 2;
     const int64_t draws = 2 * (int64_t)job_max_spp + d1 * (2 * (int64_t)job_max_spp - 1) + d2 * (3 * (int64_t)job_max_spp - 1);
     if (draws >= (int64_t)kJumpLo * kJumpHi) throw HipError{"samples per pixel too large for the sampler's jump tables", YAR_ERR_CAPACITY};
@@ -998,7 +1006,8 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     ctx->hit_ot.reserve(np);
     ctx->pk.reserve(np);
     ctx->state.reserve(np);
-    if (sequential) ctx->rng.reserve(np);
+    if (fallback) ctx->rng.reserve((size_t)max_chunk_pixels);
+    if (deep) ctx->first_parked.reserve((size_t)max_chunk_pixels);
     DevBuf<uint32_t>* qb[] = {&ctx->q_a, &ctx->q_b, &ctx->sh_path, &ctx->mi_path, &ctx->dl_path};
     for (auto* b : qb) b->reserve(np);
     ctx->mi_ndw.reserve(np);
@@ -1127,8 +1136,13 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
             for (int pass = 0; pass < passes; pass++) {
                 Chunk c = make_chunk(ci);
                 c.pass = pass;
+                c.deep = deep ? 1 : 0;
                 steps.push_back({(int)ci, pass, hc.size()});
                 hc.push_back(c);
+                if (deep) {                          // the record of the chunk's resumed paths, next to its own
+                    c.deep = 2;
+                    hc.push_back(c);
+                }
             }
         }
     }
@@ -1139,7 +1153,8 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     Paths P{};
     P.ray_o = ctx->ray_o.p; P.ray_d = ctx->ray_d.p; P.coeff = ctx->coeff.p; P.L = ctx->L.p; P.state = ctx->state.p;
     P.dl_coeff = ctx->dl_coeff.p; P.dl_light = ctx->dl_light.p; P.dl_bsdf = ctx->dl_bsdf.p; P.hit_tb = ctx->hit_tb.p;
-    P.hit_ot = ctx->hit_ot.p; P.pk = ctx->pk.p; P.rng = sequential ? ctx->rng.p : nullptr; P.radiance = ctx->radiance.p;
+    P.hit_ot = ctx->hit_ot.p; P.pk = ctx->pk.p; P.rng = fallback ? ctx->rng.p : nullptr;
+    P.first_parked = deep ? ctx->first_parked.p : nullptr; P.radiance = ctx->radiance.p;
     P.grng = guided ? ctx->grng.p : nullptr;
     P.rec = guided ? ctx->rec.p : nullptr;
     Queues q{};
@@ -1177,6 +1192,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     lc.trav_grid = ctx->cu_count * traversal_blocks_per_cu(lc, 0);
     lc.shadow_grid = ctx->cu_count * traversal_blocks_per_cu(lc, 1);
     lc.mis_grid = ctx->cu_count * traversal_blocks_per_cu(lc, 2);
+    lc.fallback = fallback;
     lc.path_grid = (int)std::max<int64_t>(1, std::min<int64_t>((max_chunk_paths + 255) / 256, (int64_t)ctx->cu_count * 8));
     if (guided) {
         lc.guided = true;
@@ -1187,8 +1203,9 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     const bool use_graph = ctx->opt.use_graph != 0 && !guided;
     Chunk* slot = ctx->chunk_slot.p;
 
-    // polling slots: one per iteration (eager) or per (chunk, pass) completion check (graph)
-    const size_t poll_n = std::max<size_t>(hc.size() + 1, (size_t)iters + 1) + 1;
+    // polling slots: a ring of four for the iterations, one per (chunk, pass) completion check (graph) and
+    // one for the training-record count
+    const size_t poll_n = 4 + hc.size() + 1;
     if (ctx->h_poll_n < poll_n) {
         if (ctx->h_poll) (void)hipHostFree(ctx->h_poll);
         ctx->h_poll = nullptr;
@@ -1220,7 +1237,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     KernelTimer kt;
     kt.on = ctx->opt.enable_timing != 0 && !use_graph;
     kt.s = s;
-    std::vector<hipEvent_t> ev((size_t)iters + 1);
+    std::vector<hipEvent_t> ev(4);
     for (auto& e : ev) HIPX(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     hipEvent_t e0, e1;
     HIPX(hipEventCreate(&e0));
@@ -1229,26 +1246,18 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     bool loop_ok = true;
     int64_t train_records = 0;
     double train_seconds = 0.0, train_nats = 0.0;
-    auto run_pass_loop = [&](const Step& sp) {
-        const Chunk& c = hc[sp.hc];
-        if (use_graph) {
-            HIPX(hipGraphLaunch(ctx->graph, s));
-            // the active list the last iteration wrote must be empty
-            HIPX(hipMemcpyAsync(hp + sp.hc, ctx->counts.p + (iters & 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-            return;
-        }
-        kt.begin(4);
-        launch_raygen(slot, c.n_paths, P, q, s);
-        kt.end();
-        // Queue kernels take their counts from device memory; the host reads each iteration's
-        // active count asynchronously and stops enqueueing two iterations after it saw zero.
-        int it = 0;
-        for (; it < iters; it++) {
+    // Bounce iterations from parity 0 on.  Queue kernels take their counts from device memory; the host
+    // reads each iteration's active count asynchronously and stops enqueueing two iterations after it saw
+    // zero.  False when `limit` iterations leave paths.
+    auto run_iterations = [&](int64_t limit) {
+        constexpr int kRing = 4;                     // polling slots and events in use at a time: three
+        int64_t it = 0;
+        for (; it < limit; it++) {
             if (it >= 2) {
-                HIPX(hipEventSynchronize(ev[it - 2]));
-                if (hp[it - 2] == 0) break;
+                HIPX(hipEventSynchronize(ev[(it - 2) % kRing]));
+                if (hp[(it - 2) % kRing] == 0) return true;
             }
-            const int parity = it & 1;
+            const int parity = (int)(it & 1);
             if (kt.on) {
                 static const int kind_of_stage[kStageCount] = {4, 0, 1, 5, 5, 4, 2, 3, 4};
                 for (int stage = 0; stage < kStageCount; stage++) {
@@ -1259,12 +1268,33 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
             } else {
                 launch_iteration(ctx->scene, slot, P, q, parity, lc);
             }
-            HIPX(hipMemcpyAsync(hp + it, ctx->counts.p + (parity ^ 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-            HIPX(hipEventRecord(ev[it], s));
+            HIPX(hipMemcpyAsync(hp + it % kRing, ctx->counts.p + (parity ^ 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipEventRecord(ev[it % kRing], s));
         }
-        if (it == iters) {
-            HIPX(hipEventSynchronize(ev[it - 1]));
-            if (hp[it - 1] != 0) loop_ok = false;
+        HIPX(hipEventSynchronize(ev[(it - 1) % kRing]));
+        return hp[(it - 1) % kRing] == 0;
+    };
+    auto run_pass_loop = [&](const Step& sp) {
+        const Chunk& c = hc[sp.hc];
+        if (use_graph) {
+            HIPX(hipGraphLaunch(ctx->graph, s));
+            // the active list the last iteration wrote must be empty
+            HIPX(hipMemcpyAsync(hp + 4 + sp.hc, ctx->counts.p + (iters & 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        } else {
+            kt.begin(4);
+            launch_raygen(slot, c.n_paths, P, q, s);
+            kt.end();
+            if (!run_iterations(iters)) loop_ok = false;
+        }
+        if (c.deep) {
+            HIPX(hipMemcpyAsync(slot, ctx->chunks.p + sp.hc + 1, sizeof(Chunk), hipMemcpyDeviceToDevice, s));
+            kt.begin(4);
+            launch_resume(slot, c.n_pixels, P, q, s);
+            kt.end();
+            HIPX(hipMemcpyAsync(hp, ctx->counts.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipStreamSynchronize(s));
+            // a pixel's parked samples follow each other, each through at most all iterations
+            if (hp[0] != 0 && !run_iterations((int64_t)c.max_spp * (iters + 1))) loop_ok = false;
         }
     };
     auto run_film = [&](const Step& sp) {
@@ -1324,8 +1354,8 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     HIPX(hipStreamSynchronize(s));
     for (auto e : ev) (void)hipEventDestroy(e);
     if (use_graph)
-        for (size_t i = 0; i < hc.size(); i++)
-            if (hp[i] != 0) loop_ok = false;
+        for (const Step& sp : steps)
+            if (hp[4 + sp.hc] != 0) loop_ok = false;
     if (!loop_ok) throw HipError{"bounce loop did not terminate within max_light_bounces + 2 iterations"};
     double ksec[kTimerKinds];
     kt.collect(ksec);
@@ -1414,7 +1444,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     st = yar_render_stats{};
     st.gpu_seconds = gpu_ms * 1e-3;
     st.samples = samples;
-    st.closest_rays = (int64_t)(tot[16] + tot[18]);
+    st.closest_rays = (int64_t)(tot[16] - tot[21] + tot[18]);
     st.any_rays = (int64_t)tot[17];
     st.node_visits = (int64_t)(tot[0] + tot[4] + tot[8]);
     st.leaf_refs = (int64_t)(tot[1] + tot[5] + tot[9]);
@@ -1424,7 +1454,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     st.extend_leaf_refs = (int64_t)tot[1];
     st.extend_triangle_tests = (int64_t)tot[2];
     st.extend_object_visits = (int64_t)tot[3];
-    st.extend_rays = (int64_t)tot[16];
+    st.extend_rays = (int64_t)(tot[16] - tot[21]);
     st.extend_launches = (int64_t)tot[19];
     st.mis_culled_rays = (int64_t)tot[20];
     st.extend_seconds = ksec[0];

@@ -33,7 +33,8 @@ struct Paths {
     float4* hit_tb;      // closest hit: t, barycentrics
     int2* hit_ot;        // closest hit: object, global triangle
     uint2* pk;           // chunk pixel and sample index of the path
-    uint64_t* rng;       // per-pixel fallback stream (sequential sample mode only)
+    uint64_t* rng;       // per-pixel fallback stream (paths of more than ten bounces only)
+    int* first_parked;   // per chunk pixel: its first sample that waits for the fallback stream
     float4* radiance;    // final per-sample radiance of the chunk, at pix_first[pixel] + sample
     // guided form only
     uint64_t* grng;      // per-path stream: strategy choice, mixture sampling, fallback dimensions
@@ -51,7 +52,10 @@ enum : uint32_t {
     kDone = 1u << 26,         // path finished; finalize after the resolve pass
     kRecShift = 27,           // bits 27..29: training vertices recorded so far (guided form)
     kRecPending = 1u << 30,   // the newest vertex still needs its post-direct-lighting radiance
+    kParked = 1u << 31,       // the path waits for its pixel's fallback stream
 };
+// Queue entry of a path that resumes with the hit it was parked at: it needs no traversal.
+constexpr uint32_t kResumed = 1u << 31;
 
 // Work queues.  The active path list ping-pongs between two buffers; `parity` selects the input.
 // counts: [0], [1] active lists, [2] shadow, [3] mis, [4] dl, [5] film side entries,
@@ -72,7 +76,8 @@ struct Queues {
     uint32_t train_cap;
     float keep_prob;
     // [0..15] traversal counters (4 per kernel kind), [16] extend rays, [17] shadow rays, [18] mis rays,
-    // [19] extend launches, [20] MIS rays answered by the light-rectangle test (count_culls only)
+    // [19] extend launches, [20] MIS rays answered by the light-rectangle test (count_culls only),
+    // [21] parked paths (their queue entries are counted as extend rays once more)
     unsigned long long* totals;
     int count_culls;
     // Direction binning of the next iteration's active list (bin_rays = 1, 2, 3: cube-map cells of
@@ -98,7 +103,11 @@ struct Chunk {
     long long n_paths;              // paths of the current pass
     int n_pixels, max_spp;
     int d1, d2, perm_bytes;         // sample-vector dims (reference_renderer.cpp:87-99)
-    int pass, sequential;           // sequential: one sample per pixel per pass (RNG fallback)
+    // Beyond ten bounces a pixel's samples draw from one stream in sample order.  deep 1: all samples at
+    // once, each parked where it may need the stream; deep 2: the parked samples of a pixel resume one after
+    // the other.  sequential: one sample per pixel per pass (a chunk too large for its paths to be in flight)
+    int deep;
+    int pass, sequential;
     int max_bounces, rr_bounce_threshold;
     float rr_threshold, film_scale, max_component;
     // guided form: this pass traces samples [k0, k1) of every pixel, slot = pixel * (k1 - k0) + j
@@ -135,11 +144,14 @@ struct LaunchCfg {
     int path_grid;            // grid-stride grid of per-path kernels (blocks of 256)
     hipStream_t stream;
     bool guided;              // launch the guide stages
+    bool fallback;            // paths may draw from the pixel's fallback stream
     GuideNet net;
     int guide_grid;
 };
 
 void launch_sample_perms(const Chunk& host_chunk, const Chunk* dev_chunk, hipStream_t s);
+// Queues the first parked path of every pixel for iteration parity 0.
+void launch_resume(const Chunk* c, int n_pixels, const Paths& p, Queues q, hipStream_t s);
 void launch_raygen(const Chunk* c, long long n_paths_max, const Paths& p, Queues q, hipStream_t s);
 // Stages of one bounce-loop iteration, in launch order.
 enum IterStage {

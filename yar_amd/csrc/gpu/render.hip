@@ -513,9 +513,10 @@ __global__ void k_raygen(const Chunk* __restrict__ cp, Paths P, Queues q) {
             uint64_t ginc;
             P.grng[s] = pcg_seed_state(guide_stream(c, make_uint2((uint32_t)p, (uint32_t)k)), ginc);
         }
-        if (c.sequential && c.pass == 0) {
+        if (c.deep && k == 0) P.first_parked[p] = 0x7fffffff;
+        if ((c.sequential && c.pass == 0) || (c.deep && k == 0)) {
             // fallback stream: the pixel's RNG after next_pixel() drew every table value
-            P.rng[s] = pcg_jump(c.jt, ps.s0, ps.inc, sampler_draws((uint32_t)v.spp, (uint32_t)c.d1, (uint32_t)c.d2));
+            P.rng[p] = pcg_jump(c.jt, ps.s0, ps.inc, sampler_draws((uint32_t)v.spp, (uint32_t)c.d1, (uint32_t)c.d2));
         }
     }
     if (c.uniform_spp > 0 && !c.guided && !c.sequential) {
@@ -540,6 +541,37 @@ __global__ void k_zero_counts(uint32_t* counts, int n) {
 void launch_raygen(const Chunk* c, long long n_paths_max, const Paths& p, Queues q, hipStream_t s) {
     hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, q.counts, 16);
     hipLaunchKernelGGL(k_raygen, dim3((unsigned)((n_paths_max + 255) / 256)), dim3(256), 0, s, c, p, q);
+}
+
+// The pixel's next parked sample after sample k, ready to queue, or kNoSlot.
+constexpr uint32_t kNoSlot = 0xffffffffu;
+YG_INLINE uint32_t take_parked(const Chunk& c, const Paths& P, int p, int k) {
+    const uint32_t end = (uint32_t)c.pix_first[p + 1];
+    for (uint32_t s = (uint32_t)c.pix_first[p] + (uint32_t)k; s < end; s++) {
+        const uint32_t st = P.state[s];
+        if (st & kParked) {
+            P.state[s] = st & ~kParked;
+            return s | kResumed;
+        }
+    }
+    return kNoSlot;
+}
+
+__global__ void k_resume(const Chunk* __restrict__ cp, Paths P, Queues q) {
+    const Chunk& c = *cp;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t slot = kNoSlot;
+    if (p < c.n_pixels && P.first_parked[p] != 0x7fffffff) slot = take_parked(c, P, p, P.first_parked[p]);
+    uint32_t* const ctr[1] = {&q.counts[0]};
+    const bool pred[1] = {slot != kNoSlot};
+    uint32_t idx[1];
+    block_append<1>(ctr, pred, idx);
+    if (pred[0]) q.active0[idx[0]] = slot;
+}
+
+void launch_resume(const Chunk* c, int n_pixels, const Paths& p, Queues q, hipStream_t s) {
+    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, q.counts, 16);
+    hipLaunchKernelGGL(k_resume, dim3((n_pixels + 255) / 256), dim3(256), 0, s, c, p, q);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -635,13 +667,14 @@ __global__ void YG_TRAV_BOUNDS k_extend(DevScene sc, Paths P, Queues q, int pari
     with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
         trace_queue<false, COUNT>(sc, n, &q.counts[6], st, depth, cnt, cfg,
             [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
-                const uint32_t slot = in[i];
+                const uint32_t entry = in[i], slot = entry & ~kResumed;
                 o = from4(P.ray_o[slot]);
                 d = from4(P.ray_d[slot]);
-                tmax = f_inf();
-                return slot;
+                tmax = entry & kResumed ? -1.f : f_inf();        // a resumed path has its hit: no interval to search
+                return entry;
             },
             [&](uint32_t slot, const Tracer<false, COUNT>& tr) {
+                if (slot & kResumed) return;
                 const HitRec& h = tr.hit;
                 P.hit_tb[slot] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
                 P.hit_ot[slot] = make_int2(h.obj, (int)h.tri);
@@ -765,10 +798,12 @@ YG_INLINE void finalize(const Chunk& c, const Paths& P, uint2 pk, RGB L) {      
     P.radiance[c.pix_first[pk.x] + pk.y] = f4(L, 0.f);
 }
 
-// GUIDED selects the guided form's variant at compile time, so the plain kernel keeps its own
-// (smaller) register allocation.
-template <bool GUIDED, bool MIX>
+// MODE selects the guided form's variant and that of paths that may draw from the pixel's fallback stream
+// at compile time, so the plain kernel keeps its own (smaller) register allocation.
+enum ShadeMode { kPlain, kGuidedMode, kFallbackMode };
+template <int MODE, bool MIX>
 __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity) {
+    constexpr bool GUIDED = MODE == kGuidedMode, FALLBACK = MODE == kFallbackMode;
     const Chunk& c = *cp;
     const uint32_t* in = parity ? q.active1 : q.active0;
     uint32_t* out = q.bin_rays ? q.unsorted : (parity ? q.active0 : q.active1);
@@ -777,17 +812,35 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restri
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t blk = blockIdx.x * blockDim.x; blk < n; blk += stride) {
         const uint32_t i = blk + threadIdx.x;
-        const bool valid = i < n;
+        bool valid = i < n;
+        if (FALLBACK && c.deep == 1) {
+            // Park a path that goes on and may draw more values than its sample tables hold (three 1D and
+            // three 2D values of the vertex, a roulette value before and after it).
+            bool park = false;
+            if (valid) {
+                const uint32_t slot = in[i], st = P.state[slot];
+                const int c1 = (int)((st >> 8) & 0xffu), c2 = (int)((st >> 16) & 0xffu), ob = P.hit_ot[slot].x;
+                park = (c1 + (st & kDelta ? 5 : 4) > c.d1 || c2 + 3 > c.d2) && ob >= 0 && s.obj_info[ob].y < 0;
+                if (park) {
+                    const uint2 pk = P.pk[slot];
+                    P.state[slot] = st | kParked;
+                    atomicMin(&P.first_parked[pk.x], (int)pk.y);
+                    valid = false;
+                }
+            }
+            const uint64_t m = __ballot(park);
+            if (__lane_id() == 0 && m) atomicAdd(&q.totals[21], (unsigned long long)__popcll(m));
+        }
         bool want_active = false, want_shadow = false, want_mis = false, want_dl = false, want_guide = false;
         bool mis_culled = false;
         float4 g_x0, g_x1, g_x2, g_x3;
-        uint32_t slot = 0;
+        uint32_t slot = 0, next_slot = kNoSlot;      // next_slot: the queue entry of the next iteration
         V3 sh_o = v3(0, 0, 0), sh_d = v3(0, 0, 0), mi_o = v3(0, 0, 0), mi_d = v3(0, 0, 0);
         float sh_tmax = 0.f, mi_pdf = 0.f, mi_ndw = 0.f, mi_lndw = 0.f;
         RGB sh_c = rgb(0, 0, 0), mi_f = rgb(0, 0, 0);
         int mi_light = 0;
         if (valid) {
-            slot = in[i];
+            slot = FALLBACK ? in[i] & ~kResumed : in[i];
             uint32_t st = P.state[slot];
             int bounce = (int)(st & 0xffu), c1 = (int)((st >> 8) & 0xffu), c2 = (int)((st >> 16) & 0xffu);
             const bool delta_traced = (st & kDelta) != 0;
@@ -802,14 +855,14 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restri
             const int p = (int)pk.x, k = (int)pk.y;
             const DevView& v = c.views[c.pix_view[p]];
             const PixelSampler ps = pixel_sampler(c, p);
-            const bool seq = c.sequential != 0;
+            const bool seq = FALLBACK && (c.sequential != 0 || c.deep == 2);
             uint64_t rs = 0, rinc = 0;
             if (GUIDED && c.guided) {
                 rinc = guide_inc(c, pk);
                 rs = P.grng[slot];
             } else if (seq) {
                 rinc = ((uint64_t)stream_id(c.pixels[p], v.seed_offset) << 1u) | 1u;
-                rs = P.rng[slot];
+                rs = P.rng[p];
             }
             int nrec = (int)((st >> kRecShift) & 7u);
             auto next1 = [&]() -> float {                               // pixel_sampling.cpp:159
@@ -1267,24 +1320,26 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restri
             else if (finished) {
                 if (GUIDED && c.guided) emit_records(P, q, slot, nrec, L, rs, rinc);
                 finalize(c, P, pk, L);
+                if (FALLBACK && c.deep == 2) next_slot = take_parked(c, P, p, k + 1);
             }
             P.state[slot] = (uint32_t)bounce | ((uint32_t)c1 << 8) | ((uint32_t)c2 << 16) | flags |
                             ((uint32_t)nrec << kRecShift);
             P.coeff[slot] = f4(coeff, 0.f);
             P.L[slot] = f4(L, 0.f);
             if (GUIDED && c.guided) P.grng[slot] = rs;
-            else if (seq) P.rng[slot] = rs;
+            else if (seq) P.rng[p] = rs;
+            if (want_active) next_slot = slot;
         }
         if (q.count_culls) {
             const uint64_t m = __ballot(mis_culled);
             if (__lane_id() == 0 && m) atomicAdd(&q.totals[20], (unsigned long long)__popcll(m));
         }
         uint32_t* const ctr[4] = {n_out, &q.counts[2], &q.counts[3], &q.counts[4]};
-        const bool pred[4] = {want_active, want_shadow, want_mis, want_dl};
+        const bool pred[4] = {next_slot != kNoSlot, want_shadow, want_mis, want_dl};
         uint32_t qi[4];
         block_append<4>(ctr, pred, qi);
         const uint32_t ia = qi[0], is = qi[1], im = qi[2], id = qi[3];
-        if (want_active) out[ia] = slot;
+        if (next_slot != kNoSlot) out[ia] = next_slot;
         if (want_shadow) {
             q.shadow_path[is] = slot;
             q.shadow_o[is] = f4(sh_o, sh_tmax);
@@ -1396,7 +1451,7 @@ __global__ void k_guide_sample(DevScene s, const Chunk* __restrict__ cp, Paths P
 }
 
 // Resolve: L += coeff * N * (light half + BSDF half) (path_tracing.cpp:56-57, direct_lighting.cpp:551)
-__global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q) {
+__global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity) {
     const uint32_t n = q.counts[4];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -1419,6 +1474,10 @@ __global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Que
                 P.grng[slot] = rs;
             }
             finalize(c, P, pk, L);
+            if (c.deep == 2) {
+                const uint32_t next = take_parked(c, P, (int)pk.x, (int)pk.y + 1);
+                if (next != kNoSlot) (parity ? q.active0 : q.active1)[atomicAdd(&q.counts[parity ^ 1], 1u)] = next;
+            }
         }
         P.state[slot] = st & ~(kPendingDL | kDone | kRecPending);
     }
@@ -1468,7 +1527,7 @@ __global__ __launch_bounds__(256) void k_bin_local(Paths P, Queues q, int parity
         __syncthreads();
         for (int j = t; j < m; j += 256) {
             const uint32_t slot = q.unsorted[base + j];
-            const uint32_t key = dir_cell<C>(P.ray_d[slot]);
+            const uint32_t key = dir_cell<C>(P.ray_d[slot & ~kResumed]);
             s_slot[j] = slot;
             s_key[j] = (uint16_t)key;
             atomicAdd(&s_cur[key], 1u);
@@ -1553,10 +1612,11 @@ void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p,
     case kStageExtend: YG_LAUNCH_TRAV(k_extend, cfg.trav_grid, sc, p, q, parity); break;
     case kStageShade:
         // scenes with mix materials take the variant whose BSDF code evaluates sub-materials
-        if (cfg.guided && sc.has_mix) hipLaunchKernelGGL((k_shade<true, true>), dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity);
-        else if (cfg.guided) hipLaunchKernelGGL((k_shade<true, false>), dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity);
-        else if (sc.has_mix) hipLaunchKernelGGL((k_shade<false, true>), dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity);
-        else hipLaunchKernelGGL((k_shade<false, false>), dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity);
+#define YG_SHADE(MODE, MIX) hipLaunchKernelGGL((k_shade<MODE, MIX>), dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity)
+        if (cfg.guided) { if (sc.has_mix) YG_SHADE(kGuidedMode, true); else YG_SHADE(kGuidedMode, false); }
+        else if (cfg.fallback) { if (sc.has_mix) YG_SHADE(kFallbackMode, true); else YG_SHADE(kFallbackMode, false); }
+        else { if (sc.has_mix) YG_SHADE(kPlain, true); else YG_SHADE(kPlain, false); }
+#undef YG_SHADE
         break;
     case kStageShadow: YG_LAUNCH_TRAV(k_shadow, cfg.shadow_grid, sc, p, q); break;
     case kStageMis: YG_LAUNCH_TRAV(k_mis, cfg.mis_grid, sc, p, q); break;
@@ -1567,7 +1627,7 @@ void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p,
         if (cfg.guided)
             hipLaunchKernelGGL(k_guide_sample, dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity);
         break;
-    case kStageResolve: hipLaunchKernelGGL(k_resolve, dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q); break;
+    case kStageResolve: hipLaunchKernelGGL(k_resolve, dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity); break;
     default: break;
     }
 }
