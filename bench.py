@@ -250,7 +250,7 @@ def main():
     scene = _scene(args.config, args.scale, args.seed)
     t_load = time.perf_counter() - t0
     ntri = scene.triangle_count()
-    opts = dict(enable_timing=1)
+    opts = {}
     if args.block:
         opts["block_size"] = args.block
     if args.stack:
@@ -286,12 +286,18 @@ def main():
     value = samples / (elapsed / args.steps) / 1e6
     rays_per_s = rays / (elapsed / args.steps)
 
-    ext_sec = sum(s.extend_seconds for s in stats) / len(stats)
-    ext_launches = stats[0].extend_launches
+    # per-kernel times: the same render with the traversal's path, shadow and MIS rays in launches of their
+    # own between HIP events (the timed steps run them as one launch per bounce); the second of two
+    tctx = yar_amd.Context(scene, **dict(opts, enable_timing=1))
+    for _ in range(2):
+        _, _, _, ts = tctx.render(0, want_film=False)
+    tctx.close()
+    ext_sec = ts.extend_seconds
+    ext_launches = ts.extend_launches
     roofline = None
     culled = None
     if not args.no_counters:
-        cctx = yar_amd.Context(scene, **dict(opts, enable_timing=0, enable_counters=1))
+        cctx = yar_amd.Context(scene, **dict(opts, enable_counters=1))
         _, _, _, cs = cctx.render(0, want_film=False)
         cctx.close()
         culled = cs.mis_culled_rays
@@ -308,7 +314,7 @@ def main():
             counters = json.load(open(cpath))
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                    "kernel": "k_extend (closest-hit kd traversal of path rays)",
+                    "kernel": "k_trace (kd traversal) of path rays, launched alone",
                     "limiter": "instruction issue: dependent kd-node loads under SIMD divergence (HBM traffic "
                                "and bandwidth are far below peak; see counters)",
                     "counters": counters,
@@ -351,10 +357,10 @@ def main():
         "rays_per_sample": round(rays / samples, 3),
         "gpu_ms_per_step": round(sum(s.gpu_seconds for s in stats) / len(stats) * 1e3, 2),
         "kernel_ms_per_step": {"extend": round(ext_sec * 1e3, 2),
-                               "shade": round(sum(s.shade_seconds for s in stats) / len(stats) * 1e3, 2),
-                               "shadow": round(sum(s.shadow_seconds for s in stats) / len(stats) * 1e3, 2),
-                               "mis": round(sum(s.mis_seconds for s in stats) / len(stats) * 1e3, 2),
-                               "other": round(sum(s.other_seconds for s in stats) / len(stats) * 1e3, 2)},
+                               "shade": round(ts.shade_seconds * 1e3, 2),
+                               "shadow": round(ts.shadow_seconds * 1e3, 2),
+                               "mis": round(ts.mis_seconds * 1e3, 2),
+                               "other": round(ts.other_seconds * 1e3, 2)},
         "roofline": roofline,
         "cpu_baseline": cpu,
     }

@@ -245,7 +245,8 @@ typedef struct yar_gpu_options {
     int32_t traversal_stack_depth;      /* short-stack entries per tree level, 0 = 8 (kd-restart beyond) */
     int32_t enable_counters;            /* count node visits / triangle tests per ray */
     int32_t use_graph;                  /* capture the bounce loop in a hipGraph */
-    int32_t enable_timing;              /* per-kernel HIP-event timing in yar_render_stats */
+    int32_t enable_timing;              /* per-kernel HIP-event timing in yar_render_stats: path, shadow and MIS rays
+                                           are then traced by launches of their own (one launch otherwise) */
     int32_t stack_mode;                 /* traversal stack storage: 0 = default, 1 = LDS, 2 = private */
     int32_t lane_refill;                /* idle lanes at which a traversal wave takes new rays: 0 = 24, 1 = 16, 2 = 64 (whole batches) */
     int32_t disable_mis_cull;           /* 1 = trace every MIS BSDF ray (no analytic light-rectangle test) */

@@ -310,7 +310,8 @@ struct yar_gpu_ctx {
         lc.priv_stack = opt.stack_mode == 2;
         lc.refill = opt.lane_refill == 1 ? 16 : opt.lane_refill == 2 ? 64 : 24;
         lc.counters = opt.enable_counters != 0;
-        lc.trav_grid = lc.shadow_grid = lc.mis_grid = 1;
+        lc.trav_grid = 1;
+        lc.split_kinds = opt.enable_counters != 0 || opt.enable_timing != 0;
         lc.path_grid = 1;
         lc.stream = stream;
         lc.guided = false;
@@ -855,8 +856,9 @@ static DevView make_dev_view(const yar_view& v, int tile_base) {
 }
 
 // Bounce-loop iterations that always suffice: every shade pass raises a path's bounce count by at
-// least one except the first pass after a delta (glass) event, and paths end at max_light_bounces.
-static int loop_iterations(int max_bounces) { return std::max(1, max_bounces) + 2; }
+// least one except the first pass after a delta (glass) event, and paths end at max_light_bounces; the
+// direct light of the last vertices is traced and added by one more.
+static int loop_iterations(int max_bounces) { return std::max(1, max_bounces) + 3; }
 
 // Guided render: the learned proposal, its pass schedule and training-record storage.
 struct GuidedRun {
@@ -1189,9 +1191,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         f.m2 = ctx->m2.p;
     }
     LaunchCfg lc = ctx->launch_cfg();
-    lc.trav_grid = ctx->cu_count * traversal_blocks_per_cu(lc, 0);
-    lc.shadow_grid = ctx->cu_count * traversal_blocks_per_cu(lc, 1);
-    lc.mis_grid = ctx->cu_count * traversal_blocks_per_cu(lc, 2);
+    lc.trav_grid = ctx->cu_count * traversal_blocks_per_cu(lc);
     lc.fallback = fallback;
     lc.path_grid = (int)std::max<int64_t>(1, std::min<int64_t>((max_chunk_paths + 255) / 256, (int64_t)ctx->cu_count * 8));
     if (guided) {
@@ -1203,9 +1203,9 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     const bool use_graph = ctx->opt.use_graph != 0 && !guided;
     Chunk* slot = ctx->chunk_slot.p;
 
-    // polling slots: a ring of four for the iterations, one per (chunk, pass) completion check (graph) and
+    // polling slots: a ring of four times 16 counters for the iterations, one per (chunk, pass) completion check (graph) and
     // one for the training-record count
-    const size_t poll_n = 4 + hc.size() + 1;
+    const size_t poll_n = 64 + hc.size() + 1;
     if (ctx->h_poll_n < poll_n) {
         if (ctx->h_poll) (void)hipHostFree(ctx->h_poll);
         ctx->h_poll = nullptr;
@@ -1247,19 +1247,23 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     int64_t train_records = 0;
     double train_seconds = 0.0, train_nats = 0.0;
     // Bounce iterations from parity 0 on.  Queue kernels take their counts from device memory; the host
-    // reads each iteration's active count asynchronously and stops enqueueing two iterations after it saw
-    // zero.  False when `limit` iterations leave paths.
+    // reads each iteration's counts asynchronously and stops enqueueing two iterations after it saw neither
+    // active paths nor direct light to add.  False when `limit` iterations leave any.
     auto run_iterations = [&](int64_t limit) {
         constexpr int kRing = 4;                     // polling slots and events in use at a time: three
+        auto idle = [&](int64_t it) {
+            const uint32_t* c = hp + (it % kRing) * 16;
+            return c[(it & 1) ^ 1] == 0 && c[light_count_base((int)(it & 1)) + 2] == 0;
+        };
         int64_t it = 0;
         for (; it < limit; it++) {
             if (it >= 2) {
                 HIPX(hipEventSynchronize(ev[(it - 2) % kRing]));
-                if (hp[(it - 2) % kRing] == 0) return true;
+                if (idle(it - 2)) return true;
             }
             const int parity = (int)(it & 1);
             if (kt.on) {
-                static const int kind_of_stage[kStageCount] = {4, 0, 1, 5, 5, 4, 2, 3, 4};
+                static const int kind_of_stage[kStageCount] = {4, 0, 2, 3, 4, 1, 5, 5, 4};
                 for (int stage = 0; stage < kStageCount; stage++) {
                     kt.begin(kind_of_stage[stage]);
                     launch_stage(stage, ctx->scene, slot, P, q, parity, lc);
@@ -1268,18 +1272,18 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
             } else {
                 launch_iteration(ctx->scene, slot, P, q, parity, lc);
             }
-            HIPX(hipMemcpyAsync(hp + it % kRing, ctx->counts.p + (parity ^ 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipMemcpyAsync(hp + (it % kRing) * 16, ctx->counts.p, 16 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             HIPX(hipEventRecord(ev[it % kRing], s));
         }
         HIPX(hipEventSynchronize(ev[(it - 1) % kRing]));
-        return hp[(it - 1) % kRing] == 0;
+        return idle(it - 1);
     };
     auto run_pass_loop = [&](const Step& sp) {
         const Chunk& c = hc[sp.hc];
         if (use_graph) {
             HIPX(hipGraphLaunch(ctx->graph, s));
             // the active list the last iteration wrote must be empty
-            HIPX(hipMemcpyAsync(hp + 4 + sp.hc, ctx->counts.p + (iters & 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipMemcpyAsync(hp + 64 + sp.hc, ctx->counts.p + (iters & 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         } else {
             kt.begin(4);
             launch_raygen(slot, c.n_paths, P, q, s);
@@ -1355,7 +1359,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     for (auto e : ev) (void)hipEventDestroy(e);
     if (use_graph)
         for (const Step& sp : steps)
-            if (hp[4 + sp.hc] != 0) loop_ok = false;
+            if (hp[64 + sp.hc] != 0) loop_ok = false;
     if (!loop_ok) throw HipError{"bounce loop did not terminate within max_light_bounces + 2 iterations"};
     double ksec[kTimerKinds];
     kt.collect(ksec);

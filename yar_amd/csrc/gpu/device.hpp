@@ -286,17 +286,16 @@ struct PrivStack {
 // Cap on a wave's turns, which only guarantees that every wave terminates; real trees need far fewer.
 constexpr uint32_t kMaxTurns = 1u << 28;
 
-template <bool ANY, bool COUNT>
+template <bool COUNT>
 struct Tracer {
     enum : uint32_t { kDone = 0, kObject = 1, kTriangle = 2, kDescend = 3, kLeafDone = 4 };
     // Interior nodes a lane descends per turn (a constant, so the steps are unrolled): 2, 3, 4 and 6 took
     // 85, 83.9, 83.5 and 87 ms on the 1024x1024 frame of the 2.2M-triangle scene.
     static constexpr int kDescents = 4;
     V3 o, d, inv;                   // world ray
-    float tmax_in;
-    HitRec hit;                     // hit.t bounds the query (any hit: stays at tmax)
+    HitRec hit;                     // hit.t bounds the query (any hit: stays at tmax), hit.obj >= 0 once hit
     uint32_t phase;
-    bool in_mesh, found_any;
+    bool in_mesh, any;
     // current level: ray origin and reciprocal direction, node words, ray interval, its exit, restart point
     // and the stack's top and bottom (entries are numbered as pushed; those from bottom on are live)
     V3 co, ci;
@@ -313,10 +312,9 @@ struct Tracer {
     float sx, sy, sz;
 
     // A ray that misses the scene bounds is complete at once (phase kDone).
-    YG_INLINE void start(const DevScene& s, V3 o_, V3 d_, float tmax_) {
-        o = o_; d = d_; tmax_in = tmax_;
+    YG_INLINE void start(const DevScene& s, V3 o_, V3 d_, float tmax_, bool any_) {
+        o = o_; d = d_; any = any_;
         hit.t = tmax_; hit.obj = -1; hit.tri = 0; hit.b = v3(0, 0, 0);
-        found_any = false;
         const bool inside = slab(s.scene_lo, s.scene_hi, o, d, quick_direction(d), inv, tmin, tmax);
         t1 = tmax;
         node_x = s.root.x; node_y = s.root.y; restart_t = -1.f; top = bottom = 0;
@@ -325,8 +323,7 @@ struct Tracer {
         phase = inside && hit.t > tmin ? kDescend : kDone;
     }
 
-    // closest hit: hit.t < tmax_in; any hit: found_any
-    YG_INLINE bool result() const { return ANY ? found_any : hit.t < tmax_in; }
+    YG_INLINE bool result() const { return hit.obj >= 0; }
 
     // One interior node on the way down: to a child, pushing the far one when the ray straddles the
     // split, as KdTree::intersect's inner loop (kdtree.cpp:245-290).  Both children are requested before
@@ -457,14 +454,11 @@ struct Tracer {
         if (COUNT) cnt.tri_tests++;
         V3 b;
         const float t = watertight(co, kz, sx, sy, sz, p0, p1, p2, b);
-        if (ANY ? !(t >= hit.t) : t < hit.t) {
+        if (any ? !(t >= hit.t) : t < hit.t) {
             if (!degenerate(p0, p1, p2)) {
-                if (ANY) {
-                    found_any = true;
-                    phase = kDone;
-                } else {
-                    hit.t = t; hit.tri = ti; hit.b = b; hit.obj = (int)oi;
-                }
+                if (!any) hit.t = t;
+                hit.tri = ti; hit.b = b; hit.obj = (int)oi;
+                if (any) phase = kDone;
             }
         }
     }
@@ -492,10 +486,10 @@ struct Tracer {
 };
 
 // Runs one query per calling lane to completion.
-template <bool ANY, bool COUNT, class Stack>
-YG_INLINE bool trace(const DevScene& s, V3 o, V3 d, float tmax_in, HitRec& hit, Stack& st, int depth, TravCounters& cnt) {
-    Tracer<ANY, COUNT> tr;
-    tr.start(s, o, d, tmax_in);
+template <bool COUNT, class Stack>
+YG_INLINE bool trace(const DevScene& s, V3 o, V3 d, float tmax_in, bool any, HitRec& hit, Stack& st, int depth, TravCounters& cnt) {
+    Tracer<COUNT> tr;
+    tr.start(s, o, d, tmax_in, any);
     for (uint32_t turn = 0; turn < kMaxTurns; turn++) {
         if (__ballot(tr.phase != tr.kDone) == 0ull) break;
         tr.turn(s, st, depth, cnt);
@@ -503,7 +497,6 @@ YG_INLINE bool trace(const DevScene& s, V3 o, V3 d, float tmax_in, HitRec& hit, 
     hit = tr.hit;
     return tr.result();
 }
-
 
 // ---- PCG32 (third-party/pcg/pcg_basic.c:46-75) ------------------------------------------
 constexpr uint64_t kPcgMult = 6364136223846793005ULL;

@@ -58,9 +58,10 @@ enum : uint32_t {
 constexpr uint32_t kResumed = 1u << 31;
 
 // Work queues.  The active path list ping-pongs between two buffers; `parity` selects the input.
-// counts: [0], [1] active lists, [2] shadow, [3] mis, [4] dl, [5] film side entries,
-//         [6] [7] [8] work-fetch cursors of extend, shadow and mis, [9] guide queries,
-//         [10] training records.
+// counts: [0], [1] active lists, [2] shadow, [3] mis, [4] dl of even iterations, [12] [13] [14] of odd
+//         ones, [5] film side entries, [6] [7] [8] work-fetch cursors of the traversal (path rays or all,
+//         shadow rays, MIS rays launched alone), [9] guide queries, [10] training records.
+__host__ __device__ inline int light_count_base(int parity) { return parity ? 12 : 2; }
 struct Queues {
     uint32_t* active0;
     uint32_t* active1;
@@ -139,8 +140,8 @@ struct LaunchCfg {
     bool priv_stack;          // stacks in private (scratch) memory instead of LDS
     int refill;               // idle lanes at which a wave of a persistent traversal kernel takes new rays
     bool counters;
-    int trav_grid;            // persistent traversal grids (blocks): k_extend, k_shadow, k_mis
-    int shadow_grid, mis_grid;
+    int trav_grid;            // grid of the persistent traversal kernel (blocks)
+    bool split_kinds;         // path, shadow and MIS rays in launches of their own (timed and counted renders)
     int path_grid;            // grid-stride grid of per-path kernels (blocks of 256)
     hipStream_t stream;
     bool guided;              // launch the guide stages
@@ -155,14 +156,14 @@ void launch_resume(const Chunk* c, int n_pixels, const Paths& p, Queues q, hipSt
 void launch_raygen(const Chunk* c, long long n_paths_max, const Paths& p, Queues q, hipStream_t s);
 // Stages of one bounce-loop iteration, in launch order.
 enum IterStage {
-    kStageReset, kStageExtend, kStageShade, kStageGuideForward, kStageGuideSample, kStageBin, kStageShadow, kStageMis,
-    kStageResolve, kStageCount
+    kStageReset, kStageExtend, kStageShadow, kStageMis, kStageResolve, kStageShade, kStageGuideForward, kStageGuideSample,
+    kStageBin, kStageCount
 };
 void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, const LaunchCfg& cfg);
 void launch_iteration(const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, const LaunchCfg& cfg);
 void launch_film(const Chunk* c, int n_pixels, const Paths& p, FilmParams f, Queues q, hipStream_t s);
 void launch_trace_rays(const DevScene& sc, const float4* rays, int64_t n, int any, float4* out_tb, int2* out_ot,
                        unsigned long long* totals, const LaunchCfg& cfg);
-int traversal_blocks_per_cu(const LaunchCfg& cfg, int kernel);
+int traversal_blocks_per_cu(const LaunchCfg& cfg);
 
 }  // namespace yg

@@ -1,7 +1,7 @@
 // render.hip - wavefront path-tracer kernels for gfx950 (CDNA4).
 //
 // One path per work item; the bounce loop is split into queue-driven kernels:
-//   sample_table -> raygen -> [reset -> extend -> shade -> shadow, mis -> resolve]* -> film
+//   sample_table -> raygen -> [reset -> trace -> resolve -> shade]* -> film
 // Queue kernels read their work counts from device memory and traversal kernels fetch work in
 // wave-sized batches from a device cursor, so an iteration needs no host round trip and the whole
 // bounce loop can be captured in a hipGraph.  Each kernel restates one part of the reference
@@ -575,9 +575,8 @@ void launch_resume(const Chunk* c, int n_pixels, const Paths& p, Queues q, hipSt
 }
 
 // ---------------------------------------------------------------------------------------------
-// Traversal kernels: extend (closest hit for path rays), shadow (any hit), mis (closest hit for
-// BSDF-sampled light rays, direct_lighting.cpp:163-191).  Persistent: each wave fetches 64 rays
-// at a time from a device cursor until the queue is drained.
+// Traversal: closest hits of path rays, occlusion of light rays, closest hits of BSDF-sampled light rays
+// (direct_lighting.cpp:163-191), by persistent waves.
 // ---------------------------------------------------------------------------------------------
 struct StackCfg { int depth, refill; };
 
@@ -605,11 +604,11 @@ YG_INLINE void with_stacks(StackCfg cfg, Body body) {
 // A queue of less than a batch per wave is spread over all waves: one ray's chain of dependent loads and
 // branches is what such a launch lasts, and in a wave of its own a ray does not wait for 63 others
 // (64x64 tile at 4 spp: 2.7 to 1.7 ms per render).
-// setup(index, o, d, tmax) returns the payload finish(payload, tracer) receives.
-template <bool ANY, bool COUNT, class Stack, class Setup, class Finish>
+// setup(index, o, d, tmax, any) returns the payload finish(payload, tracer) receives.
+template <bool COUNT, class Stack, class Setup, class Finish>
 YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Stack& st, int depth, TravCounters& cnt,
                            StackCfg cfg, Setup setup, Finish finish) {
-    Tracer<ANY, COUNT> tr;
+    Tracer<COUNT> tr;
     tr.phase = tr.kDone;
     const uint32_t wpb = (blockDim.x + 63u) >> 6;
     const uint32_t waves = gridDim.x * wpb;
@@ -638,8 +637,9 @@ YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Sta
                 if (tr.phase == tr.kDone && i < end) {
                     V3 o, d;
                     float tmax;
-                    payload = setup(i, o, d, tmax);
-                    tr.start(sc, o, d, tmax);
+                    bool any;
+                    payload = setup(i, o, d, tmax, any);
+                    tr.start(sc, o, d, tmax, any);
                     has = true;
                 }
                 next = min(next + (uint32_t)n_idle, end);
@@ -655,114 +655,114 @@ YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Sta
 // sixth wave needs 80, spills 28 B in k_extend and gains nothing).  Blocks of at most 256 threads.
 #define YG_TRAV_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 
+// A BSDF-sampled light ray's contribution (direct_lighting.cpp:163-191 and its sphere, mesh and environment
+// counterparts) once its closest hit is known.
+YG_INLINE void finish_mis(const DevScene& sc, const Paths& P, const Queues& q, uint32_t i, const HitRec& h, bool found) {
+    const float4 o4 = q.mis_o[i], d4 = q.mis_d[i];
+    const int light = (int)fbits(o4.w);
+    if (!found && light == sc.n_rects + sc.n_spheres + sc.n_mesh_lights) {
+        // environment light: the BSDF sample counts when nothing blocks it (direct_lighting.cpp:355-381)
+        const float4 f4v = q.mis_f[i];
+        const float bpdf = f4v.w;
+        const float w = power_heuristic(bpdf, d4.w);
+        const RGB contrib = (rgb4(sc.env->L) * rgb4(f4v)) * (w * fabsf(q.mis_ndw[i]) / bpdf);
+        P.dl_bsdf[q.mis_path[i]] = f4(contrib, 0.f);
+    } else if (found && sc.obj_info[h.obj].y == light) {
+        float lpdf;
+        RGB Le;
+        if (light < sc.n_rects) {
+            const DevRect L = sc.rects[light];
+            const float4 v0 = sc.tri_verts[3 * (size_t)h.tri], v1 = sc.tri_verts[3 * (size_t)h.tri + 1],
+                         v2 = sc.tri_verts[3 * (size_t)h.tri + 2];
+            // mesh-space hit point, as Triangle_Mesh::get_position (direct_lighting.cpp:181)
+            const V3 p = h.b.x * from4(v0) + h.b.y * from4(v1) + h.b.z * from4(v2);
+            const float dd = length(p - from4(o4));
+            const float lndw = d4.w;
+            lpdf = (dd * dd) / (L.size.x * L.size.y * lndw);
+            Le = rgb4(L.L);
+        } else if (light < sc.n_rects + sc.n_spheres) {
+            lpdf = d4.w;                                // the cone pdf (direct_lighting.cpp:247)
+            Le = rgb4(sc.spheres[light - sc.n_rects].L);
+        } else {
+            // Diffuse_Triangle_Mesh_Light_Sampler::pdf (light_sampling.cpp:163-184); a hit on
+            // the emitter's back has pdf 0 and keeps the full BSDF-sample weight, as there
+            const DevMeshLight ML = sc.mesh_lights[light - sc.n_rects - sc.n_spheres];
+            V3 lp, ln;
+            mesh_light_point(sc, h.tri, h.b, lp, ln);
+            const float lndw = dot(ln, -from4(d4));
+            lpdf = lndw <= 0.f ? 0.f : (h.t * h.t) / (lndw * ML.area);
+            Le = rgb4(ML.L);
+        }
+        const float4 f4v = q.mis_f[i];
+        const float bpdf = f4v.w;
+        const float w = power_heuristic(bpdf, lpdf);
+        const RGB contrib = (Le * rgb4(f4v)) * (w * fabsf(q.mis_ndw[i]) / bpdf);
+        P.dl_bsdf[q.mis_path[i]] = f4(contrib, 0.f);
+    }
+}
+
+// Traversal of one bounce iteration: closest hits of its path rays and, of the vertices the iteration
+// before shaded, the occlusion of light rays and the closest hits of BSDF-sampled light rays.  None of the
+// three waits for another, so they run as one queue: a launch ends with its longest ray, and one launch
+// has one such tail where three had three (637x359 at 4 spp of the 2.2M-triangle scene: 8.0 to 5.7 ms per
+// render, 1024x1024 at 64 spp: 83.8 to 79.2 ms).  `kinds` selects queues (bit 0 path, 1 shadow, 2 MIS
+// rays); timed and counted renders launch them one by one.
+constexpr uint32_t kKindShift = 30, kPathRay = 0u << kKindShift, kShadowRay = 1u << kKindShift, kMisRay = 2u << kKindShift;
 template <bool COUNT, bool PRIV>
-__global__ void YG_TRAV_BOUNDS k_extend(DevScene sc, Paths P, Queues q, int parity, StackCfg cfg) {
+__global__ void YG_TRAV_BOUNDS k_trace(DevScene sc, Paths P, Queues q, int parity, int kinds, StackCfg cfg) {
     const uint32_t* in = parity ? q.active1 : q.active0;
-    const uint32_t n = q.counts[parity];
+    const uint32_t* light_counts = q.counts + light_count_base(parity ^ 1);
+    const uint32_t n_path = kinds & 1 ? q.counts[parity] : 0u, n_shadow = kinds & 2 ? light_counts[0] : 0u,
+                   n_mis = kinds & 4 ? light_counts[1] : 0u;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        atomicAdd(&q.totals[16], (unsigned long long)n);
-        atomicAdd(&q.totals[19], 1ull);
+        if (kinds & 1) {
+            atomicAdd(&q.totals[16], (unsigned long long)n_path);
+            atomicAdd(&q.totals[19], 1ull);
+        }
+        atomicAdd(&q.totals[17], (unsigned long long)n_shadow);
+        atomicAdd(&q.totals[18], (unsigned long long)n_mis);
     }
     TravCounters cnt = {0, 0, 0, 0};
     with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
-        trace_queue<false, COUNT>(sc, n, &q.counts[6], st, depth, cnt, cfg,
-            [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
-                const uint32_t entry = in[i], slot = entry & ~kResumed;
-                o = from4(P.ray_o[slot]);
-                d = from4(P.ray_d[slot]);
-                tmax = entry & kResumed ? -1.f : f_inf();        // a resumed path has its hit: no interval to search
-                return entry;
-            },
-            [&](uint32_t slot, const Tracer<false, COUNT>& tr) {
-                if (slot & kResumed) return;
-                const HitRec& h = tr.hit;
-                P.hit_tb[slot] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
-                P.hit_ot[slot] = make_int2(h.obj, (int)h.tri);
-            });
-    });
-    flush_counters<COUNT>(q.totals, 0, cnt);
-}
-
-template <bool COUNT, bool PRIV>
-__global__ void YG_TRAV_BOUNDS k_shadow(DevScene sc, Paths P, Queues q, StackCfg cfg) {
-    const uint32_t n = q.counts[2];
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&q.totals[17], (unsigned long long)n);
-    TravCounters cnt = {0, 0, 0, 0};
-    with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
-        trace_queue<true, COUNT>(sc, n, &q.counts[7], st, depth, cnt, cfg,
-            [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
-                const float4 o4 = q.shadow_o[i];
-                o = from4(o4);
-                d = from4(q.shadow_d[i]);
-                tmax = o4.w;
-                return i;
-            },
-            [&](uint32_t i, const Tracer<true, COUNT>& tr) {
-                if (!tr.result()) P.dl_light[q.shadow_path[i]] = q.shadow_c[i];
-            });
-    });
-    flush_counters<COUNT>(q.totals, 1, cnt);
-}
-
-template <bool COUNT, bool PRIV>
-__global__ void YG_TRAV_BOUNDS k_mis(DevScene sc, Paths P, Queues q, StackCfg cfg) {
-    const uint32_t n = q.counts[3];
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&q.totals[18], (unsigned long long)n);
-    TravCounters cnt = {0, 0, 0, 0};
-    with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
-        trace_queue<false, COUNT>(sc, n, &q.counts[8], st, depth, cnt, cfg,
-            [&](uint32_t i, V3& o, V3& d, float& tmax) -> uint32_t {
+        trace_queue<COUNT>(sc, n_path + n_shadow + n_mis, &q.counts[kinds & 1 ? 6 : kinds & 2 ? 7 : 8], st, depth, cnt, cfg,
+            [&](uint32_t i, V3& o, V3& d, float& tmax, bool& any) -> uint32_t {
+                any = false;
+                tmax = f_inf();
+                if (i < n_path) {
+                    const uint32_t entry = in[i], slot = entry & ~kResumed;
+                    o = from4(P.ray_o[slot]);
+                    d = from4(P.ray_d[slot]);
+                    if (entry & kResumed) tmax = -1.f;           // a resumed path has its hit: no interval to search
+                    return entry & kResumed ? ~0u : kPathRay | slot;
+                }
+                i -= n_path;
+                if (i < n_shadow) {
+                    const float4 o4 = q.shadow_o[i];
+                    o = from4(o4);
+                    d = from4(q.shadow_d[i]);
+                    tmax = o4.w;
+                    any = true;
+                    return kShadowRay | i;
+                }
+                i -= n_shadow;
                 o = from4(q.mis_o[i]);
                 d = from4(q.mis_d[i]);
-                tmax = f_inf();
-                return i;
+                return kMisRay | i;
             },
-            [&](uint32_t i, const Tracer<false, COUNT>& tr) {
+            [&](uint32_t payload, const Tracer<COUNT>& tr) {
                 const HitRec& h = tr.hit;
-                const float4 o4 = q.mis_o[i], d4 = q.mis_d[i];
-                const int light = (int)fbits(o4.w);
-                if (!tr.result() && light == sc.n_rects + sc.n_spheres + sc.n_mesh_lights) {
-                    // environment light: the BSDF sample counts when nothing blocks it (direct_lighting.cpp:355-381)
-                    const float4 f4v = q.mis_f[i];
-                    const float bpdf = f4v.w;
-                    const float w = power_heuristic(bpdf, d4.w);
-                    const RGB contrib = (rgb4(sc.env->L) * rgb4(f4v)) * (w * fabsf(q.mis_ndw[i]) / bpdf);
-                    P.dl_bsdf[q.mis_path[i]] = f4(contrib, 0.f);
-                } else if (tr.result() && sc.obj_info[h.obj].y == light) {
-                    float lpdf;
-                    RGB Le;
-                    if (light < sc.n_rects) {
-                        const DevRect L = sc.rects[light];
-                        const float4 v0 = sc.tri_verts[3 * (size_t)h.tri], v1 = sc.tri_verts[3 * (size_t)h.tri + 1],
-                                     v2 = sc.tri_verts[3 * (size_t)h.tri + 2];
-                        // mesh-space hit point, as Triangle_Mesh::get_position (direct_lighting.cpp:181)
-                        const V3 p = h.b.x * from4(v0) + h.b.y * from4(v1) + h.b.z * from4(v2);
-                        const float dd = length(p - from4(o4));
-                        const float lndw = d4.w;
-                        lpdf = (dd * dd) / (L.size.x * L.size.y * lndw);
-                        Le = rgb4(L.L);
-                    } else if (light < sc.n_rects + sc.n_spheres) {
-                        lpdf = d4.w;                                // the cone pdf (direct_lighting.cpp:247)
-                        Le = rgb4(sc.spheres[light - sc.n_rects].L);
-                    } else {
-                        // Diffuse_Triangle_Mesh_Light_Sampler::pdf (light_sampling.cpp:163-184); a hit on
-                        // the emitter's back has pdf 0 and keeps the full BSDF-sample weight, as there
-                        const DevMeshLight ML = sc.mesh_lights[light - sc.n_rects - sc.n_spheres];
-                        V3 lp, ln;
-                        mesh_light_point(sc, h.tri, h.b, lp, ln);
-                        const float lndw = dot(ln, -from4(d4));
-                        lpdf = lndw <= 0.f ? 0.f : (h.t * h.t) / (lndw * ML.area);
-                        Le = rgb4(ML.L);
-                    }
-                    const float4 f4v = q.mis_f[i];
-                    const float bpdf = f4v.w;
-                    const float w = power_heuristic(bpdf, lpdf);
-                    const RGB contrib = (Le * rgb4(f4v)) * (w * fabsf(q.mis_ndw[i]) / bpdf);
-                    P.dl_bsdf[q.mis_path[i]] = f4(contrib, 0.f);
+                const uint32_t kind = payload & (3u << kKindShift), i = payload & ~(3u << kKindShift);
+                if (kind == kPathRay) {
+                    P.hit_tb[i] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
+                    P.hit_ot[i] = make_int2(h.obj, (int)h.tri);
+                } else if (kind == kShadowRay) {
+                    if (!tr.result()) P.dl_light[q.shadow_path[i]] = q.shadow_c[i];
+                } else if (kind == kMisRay) {
+                    finish_mis(sc, P, q, i, h, tr.result());
                 }
             });
     });
-    flush_counters<COUNT>(q.totals, 2, cnt);
+    flush_counters<COUNT>(q.totals, kinds == 2 ? 1 : kinds == 4 ? 2 : 0, cnt);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1334,7 +1334,8 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restri
             const uint64_t m = __ballot(mis_culled);
             if (__lane_id() == 0 && m) atomicAdd(&q.totals[20], (unsigned long long)__popcll(m));
         }
-        uint32_t* const ctr[4] = {n_out, &q.counts[2], &q.counts[3], &q.counts[4]};
+        uint32_t* const light = q.counts + light_count_base(parity);
+        uint32_t* const ctr[4] = {n_out, &light[0], &light[1], &light[2]};
         const bool pred[4] = {next_slot != kNoSlot, want_shadow, want_mis, want_dl};
         uint32_t qi[4];
         block_append<4>(ctr, pred, qi);
@@ -1450,9 +1451,9 @@ __global__ void k_guide_sample(DevScene s, const Chunk* __restrict__ cp, Paths P
     }
 }
 
-// Resolve: L += coeff * N * (light half + BSDF half) (path_tracing.cpp:56-57, direct_lighting.cpp:551)
+// Resolve, for the vertices the iteration before shaded: L += coeff * N * (light half + BSDF half) (path_tracing.cpp:56-57, direct_lighting.cpp:551)
 __global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity) {
-    const uint32_t n = q.counts[4];
+    const uint32_t n = q.counts[light_count_base(parity ^ 1) + 2];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const uint32_t slot = q.dl_path[i];
@@ -1476,18 +1477,19 @@ __global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Que
             finalize(c, P, pk, L);
             if (c.deep == 2) {
                 const uint32_t next = take_parked(c, P, (int)pk.x, (int)pk.y + 1);
-                if (next != kNoSlot) (parity ? q.active0 : q.active1)[atomicAdd(&q.counts[parity ^ 1], 1u)] = next;
+                uint32_t* out = q.bin_rays ? q.unsorted : (parity ? q.active0 : q.active1);     // as k_shade appends
+                if (next != kNoSlot) out[atomicAdd(&q.counts[parity ^ 1], 1u)] = next;
             }
         }
         P.state[slot] = st & ~(kPendingDL | kDone | kRecPending);
     }
 }
 
-// Resets the output counters of an iteration (a kernel, not a memset, so it can sit in a graph).
+// Resets the counters an iteration appends to (a kernel, not a memset, so it can sit in a graph).
 __global__ void k_iter_reset(uint32_t* counts, int parity) {
     const int t = threadIdx.x;
     if (t == 0) counts[parity ^ 1] = 0u;
-    else if (t >= 2 && t <= 4) counts[t] = 0u;
+    else if (t <= 3) counts[light_count_base(parity) + t - 1] = 0u;
     else if (t >= 6 && t <= 9) counts[t] = 0u;
 }
 
@@ -1584,17 +1586,12 @@ static size_t stack_lds(const LaunchCfg& cfg) {
         }                                                                                                  \
     } while (0)
 
-// Resident blocks per CU of a persistent traversal kernel (0 = k_extend, 1 = k_shadow, 2 = k_mis).
-int traversal_blocks_per_cu(const LaunchCfg& cfg, int kernel) {
+// Resident blocks per CU of the persistent traversal kernel.
+int traversal_blocks_per_cu(const LaunchCfg& cfg) {
     int nb = 0;
     const size_t shm = stack_lds(cfg);
-    hipError_t e;
-#define YG_OCC(K) (cfg.priv_stack ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (K<false, true>), cfg.block, shm) \
-                                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (K<false, false>), cfg.block, shm))
-    if (kernel == 1) e = YG_OCC(k_shadow);
-    else if (kernel == 2) e = YG_OCC(k_mis);
-    else e = YG_OCC(k_extend);
-#undef YG_OCC
+    const hipError_t e = cfg.priv_stack ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_trace<false, true>), cfg.block, shm)
+                                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_trace<false, false>), cfg.block, shm);
     if (e != hipSuccess || nb <= 0) nb = 1;
     return nb;
 }
@@ -1609,7 +1606,9 @@ void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p,
         else if (q.bin_rays == 2) hipLaunchKernelGGL(k_bin_local<4>, dim3(cfg.path_grid), dim3(256), 0, cfg.stream, p, q, parity);
         else if (q.bin_rays >= 3) hipLaunchKernelGGL(k_bin_local<8>, dim3(cfg.path_grid), dim3(256), 0, cfg.stream, p, q, parity);
         break;
-    case kStageExtend: YG_LAUNCH_TRAV(k_extend, cfg.trav_grid, sc, p, q, parity); break;
+    case kStageExtend: YG_LAUNCH_TRAV(k_trace, cfg.trav_grid, sc, p, q, parity, cfg.split_kinds ? 1 : 7); break;
+    case kStageShadow: if (cfg.split_kinds) YG_LAUNCH_TRAV(k_trace, cfg.trav_grid, sc, p, q, parity, 2); break;
+    case kStageMis: if (cfg.split_kinds) YG_LAUNCH_TRAV(k_trace, cfg.trav_grid, sc, p, q, parity, 4); break;
     case kStageShade:
         // scenes with mix materials take the variant whose BSDF code evaluates sub-materials
 #define YG_SHADE(MODE, MIX) hipLaunchKernelGGL((k_shade<MODE, MIX>), dim3(cfg.path_grid), dim3(256), 0, cfg.stream, sc, c, p, q, parity)
@@ -1618,8 +1617,6 @@ void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p,
         else { if (sc.has_mix) YG_SHADE(kPlain, true); else YG_SHADE(kPlain, false); }
 #undef YG_SHADE
         break;
-    case kStageShadow: YG_LAUNCH_TRAV(k_shadow, cfg.shadow_grid, sc, p, q); break;
-    case kStageMis: YG_LAUNCH_TRAV(k_mis, cfg.mis_grid, sc, p, q); break;
     case kStageGuideForward:
         if (cfg.guided) guide_forward_dev(cfg.net, q.guide_in, 16, &q.counts[9], q.guide_out, kGOut, cfg.guide_grid, cfg.stream);
         break;
@@ -1632,7 +1629,7 @@ void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p,
     }
 }
 
-// One bounce-loop iteration: reset -> extend -> shade -> shadow -> mis -> resolve.
+// One bounce-loop iteration: reset -> extend, shadow, mis -> resolve -> shade.
 void launch_iteration(const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, const LaunchCfg& cfg) {
     for (int stage = 0; stage < kStageCount; stage++) launch_stage(stage, sc, c, p, q, parity, cfg);
 }
@@ -1819,20 +1816,17 @@ __global__ void k_trace_rays(DevScene sc, const float4* __restrict__ rays, long 
         const float4 o4 = rays[2 * i], d4 = rays[2 * i + 1];
         HitRec h;
         with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
+            const bool found = trace<COUNT>(sc, from4(o4), from4(d4), o4.w, any != 0, h, st, depth, cnt);
             if (any) {
-                bool occ = trace<true, COUNT>(sc, from4(o4), from4(d4), o4.w, h, st, depth, cnt);
-                out_tb[i] = make_float4(occ ? 1.f : 0.f, 0.f, 0.f, 0.f);
+                out_tb[i] = make_float4(found ? 1.f : 0.f, 0.f, 0.f, 0.f);
                 out_ot[i] = make_int2(-1, -1);
+            } else if (found) {
+                const int tri_base = sc.obj_info[h.obj].w;
+                out_tb[i] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
+                out_ot[i] = make_int2(h.obj, (int)h.tri - tri_base);
             } else {
-                bool found = trace<false, COUNT>(sc, from4(o4), from4(d4), o4.w, h, st, depth, cnt);
-                if (found) {
-                    const int tri_base = sc.obj_info[h.obj].w;
-                    out_tb[i] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
-                    out_ot[i] = make_int2(h.obj, (int)h.tri - tri_base);
-                } else {
-                    out_tb[i] = make_float4(f_inf(), 0.f, 0.f, 0.f);
-                    out_ot[i] = make_int2(-1, -1);
-                }
+                out_tb[i] = make_float4(f_inf(), 0.f, 0.f, 0.f);
+                out_ot[i] = make_int2(-1, -1);
             }
         });
     }
