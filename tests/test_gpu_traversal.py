@@ -96,3 +96,37 @@ def test_deep_paths_in_flight_match_one_sample_per_pass(depth, grid, region, opt
     for img, film, var, closest, any_rays in out[1:]:
         assert np.array_equal(img, out[0][0]) and np.array_equal(film, out[0][1]) and var == out[0][2]
         assert (closest, any_rays) == (out[0][3], out[0][4])
+
+
+@pytest.mark.parametrize("objects", [2, 6, 40])
+def test_objects_in_many_scene_leaves(objects, scene_dir, oracle):
+    """Long thin boxes across each other, so every one lies in many leaves of the scene tree: a ray passes
+    over an object it searched before (the last four), and must still find the oracle's hits."""
+    rng = np.random.default_rng(objects)
+    text = ['LookAt 0 0 6 0 0 0 0 1 0', 'Camera "perspective" "float fov" [ 60 ]',
+            'Film "image" "integer xresolution" [ 64 ] "integer yresolution" [ 64 ] "string filename" "o.exr"',
+            'Sampler "stratified" "integer xsamples" [ 1 ] "integer ysamples" [ 1 ]', 'Integrator "path" "integer maxdepth" [ 3 ]',
+            'PixelFilter "box"', 'WorldBegin', 'LightSource "point" "point from" [ 0 3 3 ] "rgb I" [ 9 9 9 ]',
+            'Material "matte" "rgb Kd" [ 0.6 0.6 0.6 ]']
+    corner = np.array([[x, y, z] for x in (-1, 1) for y in (-1, 1) for z in (-1, 1)], float)
+    quads = [(0, 1, 3, 2), (4, 6, 7, 5), (0, 4, 5, 1), (2, 3, 7, 6), (0, 2, 6, 4), (1, 5, 7, 3)]
+    idx = " ".join(f"{a} {b} {c} {a} {c} {d}" for a, b, c, d in quads)
+    for k in range(objects):
+        half = np.full(3, 0.04)
+        half[k % 3] = 2.5
+        pts = corner * half + rng.uniform(-1.5, 1.5, 3)
+        text.append(f'Shape "trianglemesh" "integer indices" [ {idx} ] "point P" [ {" ".join(f"{v:.7g}" for v in pts.reshape(-1))} ]')
+    path = scene_dir / f"bars{objects}.pbrt"
+    path.write_text("\n".join(text) + "\nWorldEnd\n")
+    scene = yar_amd.Scene(str(path))
+    assert scene.desc.object_count == objects
+    rays = raygen.random_rays(scene, 1 << 15, seed=objects)
+    osc = oracle.OracleScene(scene)
+    for any_hit in (False, True):
+        if any_hit:
+            rays["tmax"] = rng.uniform(0.1, 6.0, rays.size).astype(np.float32)
+        g = yar_amd.Context(scene).trace_rays(rays, any_hit=any_hit)
+        o = osc.trace(rays, any_hit=any_hit)
+        assert np.array_equal(g["t"], o["t"])
+        if not any_hit:
+            assert np.array_equal(g["object"], o["object"]) and np.array_equal(g["triangle"], o["triangle"])
