@@ -130,3 +130,36 @@ def test_objects_in_many_scene_leaves(objects, scene_dir, oracle):
         assert np.array_equal(g["t"], o["t"])
         if not any_hit:
             assert np.array_equal(g["object"], o["object"]) and np.array_equal(g["triangle"], o["triangle"])
+
+
+@pytest.mark.parametrize("grid", [(8, 16), (3, 43), (16, 16), (1, 257), (5, 103), (32, 32), (33, 32), (64, 64)],
+                         ids=lambda g: f"{g[0] * g[1]}spp")
+def test_long_shuffle_runs(grid, c1_path, oracle):
+    """Sampler tables whose runs take 64, 32, 16, 8 and 4 lanes of a block, in bytes and 16-bit entries, in
+    whole words and not: every sampler dimension of the pixels against the oracle's paths."""
+    scene = yar_amd.Scene(c1_path)
+    ctx = yar_amd.Context(scene)
+    v = yv.with_film(ctx.view(0), 256, 256, grid, seed_offset=11, region=(120, 130, 127, 133))
+    ctx.set_views([v])
+    img, film, var, st = ctx.render(0)
+    oimg, ofilm, ovar, _, _ = oracle.OracleScene(scene).render(v)
+    rel = np.abs(img - oimg) / np.maximum(np.abs(oimg), 1e-3)
+    # a wrong permutation entry moves a sample to another stratum; device sin and cos move a path by an ulp
+    assert np.all(rel <= 1e-4, axis=-1).mean() >= 0.95
+    assert (film["weight_sum"] == ofilm["weight_sum"]).all()
+    assert abs(var - ovar) <= 1e-3 * ovar
+
+
+def test_short_and_long_runs_in_one_batch(c1_path):
+    """Views of different sample counts share a chunk's tables (runs of different lengths in one block)."""
+    scene = yar_amd.Scene(c1_path)
+    ctx = yar_amd.Context(scene)
+    base = ctx.view(0)
+    views = [yv.with_film(base, 64, 64, g, seed_offset=i, region=(20, 20, 33, 31))
+             for i, g in enumerate([(2, 2), (20, 20), (1, 1), (7, 11), (16, 17)])]
+    ctx.set_views(views)
+    imgs, var, _ = ctx.render_batch(list(range(len(views))))
+    for i, v in enumerate(views):
+        ctx.set_views([v])
+        img, _, rvar, _ = ctx.render(0, want_film=False)
+        assert np.array_equal(img, imgs[i]) and rvar == var[i]

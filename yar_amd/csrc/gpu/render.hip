@@ -284,71 +284,30 @@ YG_INLINE void sample_2d(const Chunk& c, const PixelSampler& ps, int i, int k, f
     strat2(ps, c.jt, dim2_base(spp, (uint32_t)c.d1, (uint32_t)i) + 2u * j, j, x, y);
 }
 
-// Shuffle permutations of large runs (spp > 128): one wave per (pixel, dimension) run.  The lanes
-// draw the run's swap indices in parallel (pcg32 jump-ahead to each lane's first draw, then steps
-// of 64 draws) into LDS and initialise the index array there; one lane then applies the swaps in
-// order (math.h:138-144) and the wave writes the permutation out.  Every array access is in LDS.
-template <class T>
-__global__ __launch_bounds__(64) void k_sample_perms_large(const Chunk* __restrict__ cp, int n_dims, ulonglong2 step64) {
-    extern __shared__ uint16_t big_lds[];
-    const Chunk c = *cp;
-    const long long total = (long long)c.n_pixels * n_dims;
-    const long long g = blockIdx.x;
-    if (g >= total) return;
-    const int p = (int)(g / n_dims), i = (int)(g % n_dims);
-    const DevView& v = c.views[c.pix_view[p]];
-    const int spp = v.spp;
-    uint16_t* a = big_lds;                       // index array, spp entries
-    uint16_t* jv = big_lds + c.max_spp;          // swap index of draw m (array size n = spp - m)
-    const int lane = (int)threadIdx.x;
-    uint64_t inc;
-    const uint64_t s0 = pcg_seed_state(stream_id(c.pixels[p], v.seed_offset), inc);
-    const uint32_t first = i < c.d1 ? dim1_base((uint32_t)spp, (uint32_t)i) + (uint32_t)spp
-                                    : dim2_base((uint32_t)spp, (uint32_t)c.d1, (uint32_t)(i - c.d1)) + 2u * (uint32_t)spp;
-    uint64_t st = pcg_jump(c.jt, s0, inc, first + (uint32_t)lane);
-    const uint64_t g64 = step64.y * inc;
-    for (int m = lane; m < spp - 1; m += 64) {
-        const uint32_t n = (uint32_t)(spp - m);
-        jv[m] = (uint16_t)((pcg_output(st) * (uint64_t)n) >> 32);
-        st = step64.x * st + g64;
-    }
-    for (int k = lane; k < spp; k += 64) a[k] = (uint16_t)k;
-    __syncthreads();
-    if (lane == 0) {
-        for (int m = 0; m < spp - 1; m++) {
-            const int n = spp - m;
-            const uint32_t k = jv[m];
-            const uint16_t x = a[n - 1];
-            a[n - 1] = a[k];
-            a[k] = x;
-        }
-    }
-    __syncthreads();
-    T* out = reinterpret_cast<T*>(const_cast<uint8_t*>(c.perm)) + c.pix_first[p] * (long long)n_dims + (long long)i * spp;
-    for (int k = lane; k < spp; k += 64) out[k] = (T)a[k];
-}
-
-// Shuffle permutations: one work item per (pixel, 1D or 2D dimension) applies the run's Fisher-Yates
-// swaps (math.h:138-144, the swap draws follow the run's value draws) to an index array and writes
-// the spp resulting stratum indices.  STAGED: the index arrays live in LDS as entries of type T,
-// 4 / sizeof(T) consecutive entries of one lane per 32-bit word and words laid out [word][thread], so
-// a wave's accesses fall in distinct banks while a 64-entry byte run takes 4 KB per block instead of
-// 16 KB (more resident waves to hide the serial draw-and-swap chain); the block's runs, adjacent in
-// the table, are written as one contiguous range.  Otherwise the swaps run in place on the output
-// (large spp).
+// Shuffle permutations: one lane per (pixel, 1D or 2D dimension) run applies the run's Fisher-Yates swaps
+// (math.h:138-144, the swap draws follow the run's value draws) to an index array and writes the spp
+// resulting stratum indices.  STAGED: the index arrays live in LDS as entries of type T, 4 / sizeof(T)
+// consecutive entries of one run per 32-bit word and words laid out [word][run], so a wave's accesses fall
+// in distinct banks; the block's `runs` runs, adjacent in the table, are written as one contiguous range.
+// A run is a serial chain of draws and swaps, so what counts is how many run at a time: as many as fit in
+// LDS (64 a block while that takes at most 32 KB, 16 at 1,024 entries of 2 bytes), five blocks or more per
+// CU.  One wave per run, its draws in parallel and its swaps on one lane, kept 32 runs per CU in progress
+// and took 7.3 ms against 2.2 ms on 97x89 pixels at 1,024 spp.  Otherwise (runs beyond LDS) the
+// swaps run in place on the output.
 template <class T, bool STAGED>
-__global__ void k_sample_perms(const Chunk* __restrict__ cp, int n_dims) {
+__global__ __launch_bounds__(64) void k_sample_perms(const Chunk* __restrict__ cp, int n_dims, int runs) {
     extern __shared__ uint32_t perm_lds[];
-    __shared__ long long run_off[256];
+    __shared__ long long run_off[64];
     const Chunk c = *cp;
     T* out = reinterpret_cast<T*>(const_cast<uint8_t*>(c.perm));
     const long long total = (long long)c.n_pixels * n_dims;
-    const long long g0 = (long long)blockIdx.x * blockDim.x;
+    const long long g0 = (long long)blockIdx.x * runs;
     const long long g = g0 + threadIdx.x;
+    const bool mine = (int)threadIdx.x < runs && g < total;
     const int nt = blockDim.x;
     long long off = 0;
     int spp = 0;
-    if (g < total) {
+    if (mine) {
         const int p = (int)(g / n_dims), i = (int)(g % n_dims);
         const DevView& v = c.views[c.pix_view[p]];
         spp = v.spp;
@@ -361,7 +320,7 @@ __global__ void k_sample_perms(const Chunk* __restrict__ cp, int n_dims) {
         if (STAGED) {
             constexpr int E = 4 / (int)sizeof(T);
             T* a = reinterpret_cast<T*>(perm_lds + threadIdx.x);
-            const int row = nt * E;                 // entry k at a[(k / E) * row + k % E]
+            const int row = runs * E;               // entry k at a[(k / E) * row + k % E]
             for (int k = 0; k < spp; k++) a[(k / E) * row + (k % E)] = (T)k;
             for (int n = spp; n > 1; n--) {
                 const int k = (int)(((uint64_t)pcg_next(st, inc) * (uint64_t)n) >> 32);
@@ -383,21 +342,29 @@ __global__ void k_sample_perms(const Chunk* __restrict__ cp, int n_dims) {
         }
     }
     if (!STAGED) return;
-    if (c.uniform_spp > 0 && (c.uniform_spp & 3) == 0 && sizeof(T) == 1) {
-        // every run of the chunk has the same 4-aligned length: each lane copies its own run's LDS
-        // words, which already hold four consecutive entries each, to the table
-        if (g < total) {
-            const uint32_t* a = perm_lds + threadIdx.x;
-            uint32_t* o = reinterpret_cast<uint32_t*>(out + off);
-            for (int w = 0; w < (spp >> 2); w++) o[w] = a[w * nt];
+    if (c.uniform_spp > 0 && (c.uniform_spp * sizeof(T) & 3) == 0) {
+        // every run of the chunk has the same length in whole words, which LDS holds as the table does
+        const int words = c.uniform_spp * (int)sizeof(T) / 4;
+        if (runs == 64) {                           // each lane copies its own run
+            if (mine) {
+                const uint32_t* a = perm_lds + threadIdx.x;
+                uint32_t* o = reinterpret_cast<uint32_t*>(out + off);
+                for (int w = 0; w < words; w++) o[w] = a[w * runs];
+            }
+        } else {                                    // long runs: the wave copies one after the other
+            __syncthreads();
+            const int n_runs = (int)min((long long)runs, total - g0);
+            uint32_t* o = reinterpret_cast<uint32_t*>(out + g0 * c.uniform_spp);
+            for (int r = 0; r < n_runs; r++, o += words)
+                for (int w = threadIdx.x; w < words; w += nt) o[w] = perm_lds[w * runs + r];
         }
         return;
     }
     // coalesced write-out of the block's contiguous range [run_off[0], end)
-    run_off[threadIdx.x] = g < total ? off : -1;
+    run_off[threadIdx.x] = mine ? off : -1;
     __syncthreads();
     const long long base = run_off[0];
-    const int last = (int)((total < g0 + nt ? total : g0 + nt) - g0) - 1;
+    const int last = (int)(min(total, g0 + runs) - g0) - 1;
     __shared__ long long end_s;
     if ((int)threadIdx.x == last) end_s = off + spp;
     __syncthreads();
@@ -418,38 +385,30 @@ __global__ void k_sample_perms(const Chunk* __restrict__ cp, int n_dims) {
             k = (int)(base + j - run_off[t]);
         }
         constexpr int E = 4 / (int)sizeof(T);
-        out[base + j] = reinterpret_cast<const T*>(perm_lds)[((k / E) * nt + t) * E + (k % E)];
+        out[base + j] = reinterpret_cast<const T*>(perm_lds)[((k / E) * runs + t) * E + (k % E)];
     }
 }
 
 constexpr int kPermBlock = 64;
-constexpr int kPermLargeMaxSpp = 8192;     // 2 x 2 B x spp of LDS per run (32 KB)
+constexpr int kPermLdsBytes = 32 << 10;    // of one block
+constexpr int kPermMaxSpp = 8192;          // two runs of 16 KB a block; longer ones go in place
 
 void launch_sample_perms(const Chunk& hc, const Chunk* dc, hipStream_t s) {
     const int n_dims = hc.d1 + hc.d2;
     if (n_dims == 0) return;
     const long long items = (long long)hc.n_pixels * n_dims;
-    const unsigned blocks = (unsigned)((items + kPermBlock - 1) / kPermBlock);
-    if (hc.max_spp <= 128) {
-        const int per_word = hc.perm_bytes == 1 ? 4 : 2;
-        const size_t shm = (size_t)kPermBlock * ((hc.max_spp + per_word - 1) / per_word) * sizeof(uint32_t);
-        if (hc.perm_bytes == 1) hipLaunchKernelGGL((k_sample_perms<uint8_t, true>), dim3(blocks), dim3(kPermBlock), shm, s, dc, n_dims);
-        else hipLaunchKernelGGL((k_sample_perms<uint16_t, true>), dim3(blocks), dim3(kPermBlock), shm, s, dc, n_dims);
-        return;
-    }
-    if (hc.max_spp > kPermLargeMaxSpp) {          // runs beyond the LDS of one workgroup: in place in HBM
-        if (hc.perm_bytes == 1) hipLaunchKernelGGL((k_sample_perms<uint8_t, false>), dim3(blocks), dim3(kPermBlock), 0, s, dc, n_dims);
-        else hipLaunchKernelGGL((k_sample_perms<uint16_t, false>), dim3(blocks), dim3(kPermBlock), 0, s, dc, n_dims);
-        return;
-    }
-    // one wave per run; pcg32 multiplier and increment factor of 64 steps (A_64, G_64)
-    uint64_t a64 = 1, g64 = 0;
-    for (int k = 0; k < 64; k++) { g64 = g64 * kPcgMult + 1; a64 *= kPcgMult; }
-    const ulonglong2 step64 = make_ulonglong2(a64, g64);
-    const size_t shm = (size_t)2 * hc.max_spp * sizeof(uint16_t);
-    const unsigned runs = (unsigned)items;
-    if (hc.perm_bytes == 1) hipLaunchKernelGGL((k_sample_perms_large<uint8_t>), dim3(runs), dim3(64), shm, s, dc, n_dims, step64);
-    else hipLaunchKernelGGL((k_sample_perms_large<uint16_t>), dim3(runs), dim3(64), shm, s, dc, n_dims, step64);
+    const bool staged = hc.max_spp <= kPermMaxSpp;
+    const int run_bytes = (hc.max_spp * hc.perm_bytes + 3) / 4 * 4;
+    int runs = kPermBlock;
+    while (staged && runs > 1 && runs * run_bytes > kPermLdsBytes) runs >>= 1;
+    const unsigned blocks = (unsigned)((items + runs - 1) / runs);
+    const size_t shm = staged ? (size_t)runs * run_bytes : 0;
+#define YG_PERMS(T, STAGED) hipLaunchKernelGGL((k_sample_perms<T, STAGED>), dim3(blocks), dim3(kPermBlock), shm, s, dc, n_dims, runs)
+    if (staged && hc.perm_bytes == 1) YG_PERMS(uint8_t, true);
+    else if (staged) YG_PERMS(uint16_t, true);
+    else if (hc.perm_bytes == 1) YG_PERMS(uint8_t, false);
+    else YG_PERMS(uint16_t, false);
+#undef YG_PERMS
 }
 
 // ---------------------------------------------------------------------------------------------
