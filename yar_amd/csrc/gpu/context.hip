@@ -230,13 +230,14 @@ struct yar_gpu_ctx {
     DevBuf<Chunk> chunks, chunk_slot;
     DevBuf<uint8_t> perm;                 // sampler shuffle permutations of the current chunk
     DevBuf<ulonglong2> jump_lo, jump_hi;  // pcg32 jump-ahead tables
-    DevBuf<float4> ray_o, ray_d, coeff, L, dl_coeff, dl_light, dl_bsdf, hit_tb, radiance;
+    DevBuf<float4> ray_o, ray_d, coeff, L, dl_coeff, dl_bsdf, hit_tb, radiance;
     DevBuf<int2> hit_ot;
     DevBuf<uint2> pk;
     DevBuf<uint32_t> state;
     DevBuf<uint64_t> rng;
     DevBuf<int> first_parked;
-    DevBuf<uint32_t> q_a, q_b, sh_path, mi_path, dl_path, counts, q_unsorted;
+    DevBuf<uint32_t> q_a, q_b, mi_path, dl_path, dl_shadow, counts, q_unsorted;
+    DevBuf<uint8_t> sh_seen;
     DevBuf<float4> sh_o, sh_d, sh_c, mi_o, mi_d, mi_f;
     DevBuf<float> mi_ndw;
     DevBuf<unsigned long long> totals;
@@ -279,7 +280,7 @@ struct yar_gpu_ctx {
         pairs.release(); leaf_ids.release(); pk.release();
         objs.release();
         DevBuf<float4>* b4[] = {&tri_verts, &obj_o2w, &obj_nrm, &vtx_n, &ray_o, &ray_d, &coeff, &L, &dl_coeff,
-                                &dl_light, &dl_bsdf, &hit_tb, &radiance, &sh_o, &sh_d, &sh_c, &mi_o, &mi_d,
+                                &dl_bsdf, &hit_tb, &radiance, &sh_o, &sh_d, &sh_c, &mi_o, &mi_d,
                                 &mi_f, &out_film, &side_rad, &tr_rays, &tr_tb};
         for (auto* b : b4) b->release();
         DevBuf<int4>* bi4[] = {&obj_info, &mesh_info, &tri_vidx, &side_info};
@@ -290,7 +291,8 @@ struct yar_gpu_ctx {
         spots.release(); dirs.release(); mesh_lights.release(); mesh_light_cdf.release(); spheres.release(); env.release();
         pixels.release(); pix_first.release(); dviews.release(); chunks.release(); chunk_slot.release();
         perm.release(); jump_lo.release(); jump_hi.release(); hit_ot.release(); tr_ot.release(); state.release(); rng.release();
-        DevBuf<uint32_t>* bu[] = {&q_a, &q_b, &sh_path, &mi_path, &dl_path, &counts, &q_unsorted};
+        DevBuf<uint32_t>* bu[] = {&q_a, &q_b, &mi_path, &dl_path, &dl_shadow, &counts, &q_unsorted};
+        sh_seen.release();
         for (auto* b : bu) b->release();
         mi_ndw.release(); totals.release(); out_var.release(); spill.release();
         grng.release(); rec.release(); guide_in.release(); guide_out.release(); guide_path.release(); train.release();
@@ -938,7 +940,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     // the late bounces, where most paths have ended (config 2, 1024x1024 at 64 spp: 262 Msamples/s at
     // 4M paths, 329 at 8M, 390 at 16M, 416 at 32M in two chunks, 449 at 64M in one chunk).  Guided
     // jobs revisit every chunk once per pass and keep up to 16M paths in one chunk.  Path state is
-    // about 280 B per path (plain: 14 float4 rays / throughputs / direct-lighting halves / queue
+    // about 265 B per path (plain: 13 float4 rays / throughputs / direct-lighting halves / queue
     // payloads, hit, state and 5 queue slots; 64M paths hold about 19 GB) and about 800 B guided
     // (+ training vertices, network inputs and outputs).  The default never takes more than a
     // quarter of the free device memory.
@@ -1002,7 +1004,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     ctx->perm.reserve((size_t)(max_chunk_samples * n_dims * perm_bytes));
     ctx->radiance.reserve((size_t)max_chunk_samples);
     ctx->spill.reserve((size_t)max_chunk_pixels);
-    DevBuf<float4>* pb[] = {&ctx->ray_o, &ctx->ray_d, &ctx->coeff, &ctx->L, &ctx->dl_coeff, &ctx->dl_light, &ctx->dl_bsdf,
+    DevBuf<float4>* pb[] = {&ctx->ray_o, &ctx->ray_d, &ctx->coeff, &ctx->L, &ctx->dl_coeff, &ctx->dl_bsdf,
                             &ctx->hit_tb, &ctx->sh_o, &ctx->sh_d, &ctx->sh_c, &ctx->mi_o, &ctx->mi_d, &ctx->mi_f};
     for (auto* b : pb) b->reserve(np);
     ctx->hit_ot.reserve(np);
@@ -1010,7 +1012,8 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     ctx->state.reserve(np);
     if (fallback) ctx->rng.reserve((size_t)max_chunk_pixels);
     if (deep) ctx->first_parked.reserve((size_t)max_chunk_pixels);
-    DevBuf<uint32_t>* qb[] = {&ctx->q_a, &ctx->q_b, &ctx->sh_path, &ctx->mi_path, &ctx->dl_path};
+    DevBuf<uint32_t>* qb[] = {&ctx->q_a, &ctx->q_b, &ctx->mi_path, &ctx->dl_path, &ctx->dl_shadow};
+    ctx->sh_seen.reserve(np);
     for (auto* b : qb) b->reserve(np);
     ctx->mi_ndw.reserve(np);
     ctx->counts.reserve(16);
@@ -1154,14 +1157,14 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
 
     Paths P{};
     P.ray_o = ctx->ray_o.p; P.ray_d = ctx->ray_d.p; P.coeff = ctx->coeff.p; P.L = ctx->L.p; P.state = ctx->state.p;
-    P.dl_coeff = ctx->dl_coeff.p; P.dl_light = ctx->dl_light.p; P.dl_bsdf = ctx->dl_bsdf.p; P.hit_tb = ctx->hit_tb.p;
+    P.dl_coeff = ctx->dl_coeff.p; P.dl_bsdf = ctx->dl_bsdf.p; P.hit_tb = ctx->hit_tb.p;
     P.hit_ot = ctx->hit_ot.p; P.pk = ctx->pk.p; P.rng = fallback ? ctx->rng.p : nullptr;
     P.first_parked = deep ? ctx->first_parked.p : nullptr; P.radiance = ctx->radiance.p;
     P.grng = guided ? ctx->grng.p : nullptr;
     P.rec = guided ? ctx->rec.p : nullptr;
     Queues q{};
     q.active0 = ctx->q_a.p; q.active1 = ctx->q_b.p;
-    q.shadow_path = ctx->sh_path.p; q.shadow_o = ctx->sh_o.p; q.shadow_d = ctx->sh_d.p; q.shadow_c = ctx->sh_c.p;
+    q.shadow_seen = ctx->sh_seen.p; q.dl_shadow = ctx->dl_shadow.p; q.shadow_o = ctx->sh_o.p; q.shadow_d = ctx->sh_d.p; q.shadow_c = ctx->sh_c.p;
     q.mis_path = ctx->mi_path.p; q.mis_o = ctx->mi_o.p; q.mis_d = ctx->mi_d.p; q.mis_f = ctx->mi_f.p;
     q.mis_ndw = ctx->mi_ndw.p; q.dl_path = ctx->dl_path.p; q.counts = ctx->counts.p; q.totals = ctx->totals.p;
     q.count_culls = ctx->opt.enable_counters != 0;
@@ -1223,7 +1226,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         hipGraph_t g;
         HIPX(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         launch_raygen(slot, max_chunk_paths, P, q, s);
-        for (int it = 0; it < iters; it++) launch_iteration(ctx->scene, slot, P, q, it & 1, lc);
+        for (int it = 0; it < iters; it++) launch_iteration(ctx->scene, slot, P, q, it & 1, it == 0, lc);
         HIPX(hipStreamEndCapture(s, &g));
         hipError_t e = hipGraphInstantiate(&ctx->graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
@@ -1248,8 +1251,8 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     double train_seconds = 0.0, train_nats = 0.0;
     // Bounce iterations from parity 0 on.  Queue kernels take their counts from device memory; the host
     // reads each iteration's counts asynchronously and stops enqueueing two iterations after it saw neither
-    // active paths nor direct light to add.  False when `limit` iterations leave any.
-    auto run_iterations = [&](int64_t limit) {
+    // active paths nor direct light to add.  False when `limit` iterations leave any.  `fresh`: behind raygen.
+    auto run_iterations = [&](int64_t limit, bool fresh) {
         constexpr int kRing = 4;                     // polling slots and events in use at a time: three
         auto idle = [&](int64_t it) {
             const uint32_t* c = hp + (it % kRing) * 16;
@@ -1266,11 +1269,11 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
                 static const int kind_of_stage[kStageCount] = {4, 0, 2, 3, 4, 1, 5, 5, 4};
                 for (int stage = 0; stage < kStageCount; stage++) {
                     kt.begin(kind_of_stage[stage]);
-                    launch_stage(stage, ctx->scene, slot, P, q, parity, lc);
+                    launch_stage(stage, ctx->scene, slot, P, q, parity, fresh && it == 0, lc);
                     kt.end();
                 }
             } else {
-                launch_iteration(ctx->scene, slot, P, q, parity, lc);
+                launch_iteration(ctx->scene, slot, P, q, parity, fresh && it == 0, lc);
             }
             HIPX(hipMemcpyAsync(hp + (it % kRing) * 16, ctx->counts.p, 16 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             HIPX(hipEventRecord(ev[it % kRing], s));
@@ -1288,7 +1291,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
             kt.begin(4);
             launch_raygen(slot, c.n_paths, P, q, s);
             kt.end();
-            if (!run_iterations(iters)) loop_ok = false;
+            if (!run_iterations(iters, true)) loop_ok = false;
         }
         if (c.deep) {
             HIPX(hipMemcpyAsync(slot, ctx->chunks.p + sp.hc + 1, sizeof(Chunk), hipMemcpyDeviceToDevice, s));
@@ -1298,7 +1301,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
             HIPX(hipMemcpyAsync(hp, ctx->counts.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             HIPX(hipStreamSynchronize(s));
             // a pixel's parked samples follow each other, each through at most all iterations
-            if (hp[0] != 0 && !run_iterations((int64_t)c.max_spp * (iters + 1))) loop_ok = false;
+            if (hp[0] != 0 && !run_iterations((int64_t)c.max_spp * (iters + 1), false)) loop_ok = false;
         }
     };
     auto run_film = [&](const Step& sp) {

@@ -28,8 +28,7 @@ struct Paths {
     float4* L;           // accumulated radiance
     uint32_t* state;     // bounce | c1 << 8 | c2 << 16 | flags
     float4* dl_coeff;    // throughput at the direct-lighting vertex
-    float4* dl_light;    // light-sampling half of the MIS estimate
-    float4* dl_bsdf;     // BSDF-sampling half
+    float4* dl_bsdf;     // BSDF-sampling half of the MIS estimate (vertices with a MIS ray)
     float4* hit_tb;      // closest hit: t, barycentrics
     int2* hit_ot;        // closest hit: object, global triangle
     uint2* pk;           // chunk pixel and sample index of the path
@@ -56,6 +55,8 @@ enum : uint32_t {
 };
 // Queue entry of a path that resumes with the hit it was parked at: it needs no traversal.
 constexpr uint32_t kResumed = 1u << 31;
+constexpr uint32_t kDlMis = 1u << 31;
+constexpr uint32_t kNoSlot = 0xffffffffu;
 
 // Work queues.  The active path list ping-pongs between two buffers; `parity` selects the input.
 // counts: [0], [1] active lists, [2] shadow, [3] mis, [4] dl of even iterations, [12] [13] [14] of odd
@@ -65,9 +66,12 @@ __host__ __device__ inline int light_count_base(int parity) { return parity ? 12
 struct Queues {
     uint32_t* active0;
     uint32_t* active1;
-    uint32_t* shadow_path; float4* shadow_o; float4* shadow_d; float4* shadow_c;
+    // shadow rays: contribution of the light sample, and whether the light was seen
+    float4* shadow_o; float4* shadow_d; float4* shadow_c; uint8_t* shadow_seen;
     uint32_t* mis_path; float4* mis_o; float4* mis_d; float4* mis_f; float* mis_ndw;
-    uint32_t* dl_path;
+    // vertices whose direct light is still to be added: path (| kDlMis with a MIS ray) and its shadow ray
+    // (kNoSlot without one)
+    uint32_t* dl_path; uint32_t* dl_shadow;
     uint32_t* counts;
     // guided form: continuation queries ([9] counts them) and training records ([10])
     uint32_t* guide_path;
@@ -159,8 +163,10 @@ enum IterStage {
     kStageReset, kStageExtend, kStageShadow, kStageMis, kStageResolve, kStageShade, kStageGuideForward, kStageGuideSample,
     kStageBin, kStageCount
 };
-void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, const LaunchCfg& cfg);
-void launch_iteration(const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, const LaunchCfg& cfg);
+// `first`: the iteration behind ray generation, whose paths have no state, throughput or radiance in memory
+// yet.
+void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, bool first, const LaunchCfg& cfg);
+void launch_iteration(const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, bool first, const LaunchCfg& cfg);
 void launch_film(const Chunk* c, int n_pixels, const Paths& p, FilmParams f, Queues q, hipStream_t s);
 void launch_trace_rays(const DevScene& sc, const float4* rays, int64_t n, int any, float4* out_tb, int2* out_ot,
                        unsigned long long* totals, const LaunchCfg& cfg);
