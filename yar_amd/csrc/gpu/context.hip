@@ -245,6 +245,7 @@ struct yar_gpu_ctx {
     DevBuf<double> out_var;
     DevBuf<int4> side_info;
     DevBuf<uint8_t> spill;
+    DevBuf<int2> spill_range;
     // guided form
     DevBuf<uint64_t> grng;
     DevBuf<float> rec, guide_in, guide_out;
@@ -294,7 +295,7 @@ struct yar_gpu_ctx {
         DevBuf<uint32_t>* bu[] = {&q_a, &q_b, &mi_path, &dl_path, &dl_shadow, &counts, &q_unsorted};
         sh_seen.release();
         for (auto* b : bu) b->release();
-        mi_ndw.release(); totals.release(); out_var.release(); spill.release();
+        mi_ndw.release(); totals.release(); out_var.release(); spill.release(); spill_range.release();
         grng.release(); rec.release(); guide_in.release(); guide_out.release(); guide_path.release(); train.release();
         m1.release(); m2.release();
         if (h_poll) (void)hipHostFree(h_poll);
@@ -1004,6 +1005,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     ctx->perm.reserve((size_t)(max_chunk_samples * n_dims * perm_bytes));
     ctx->radiance.reserve((size_t)max_chunk_samples);
     ctx->spill.reserve((size_t)max_chunk_pixels);
+    ctx->spill_range.reserve((size_t)max_chunk_pixels);
     DevBuf<float4>* pb[] = {&ctx->ray_o, &ctx->ray_d, &ctx->coeff, &ctx->L, &ctx->dl_coeff, &ctx->dl_bsdf,
                             &ctx->hit_tb, &ctx->sh_o, &ctx->sh_d, &ctx->sh_c, &ctx->mi_o, &ctx->mi_d, &ctx->mi_f};
     for (auto* b : pb) b->reserve(np);
@@ -1183,6 +1185,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     f.out_film = ctx->out_film.p;
     f.out_var = ctx->out_var.p;
     f.spill = ctx->spill.p;
+    f.spill_range = ctx->spill_range.p;
     f.tile_first = ctx->tile_first.p;
     f.side_rad = ctx->side_rad.p;
     f.side_info = ctx->side_info.p;

@@ -126,6 +126,7 @@ struct FilmParams {
     float4* out_film;         // per listed pixel: its Film_Tile value inside its own tile
     double* out_var;          // per listed pixel: luminance variance of its estimate
     uint8_t* spill;           // per chunk pixel: 8-neighbour footprint bits of its samples
+    int2* spill_range;        // first and last sample behind those bits (pixels with any)
     const int* tile_first;    // per (view, tile): pixel-list index of its first pixel, -1 if absent
     long long base;           // pixel-list index of the chunk's first pixel
     float4* side_rad;         // samples reaching a tile's one-pixel margin: radiance

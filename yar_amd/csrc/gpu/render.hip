@@ -757,23 +757,67 @@ YG_INLINE void finalize(const Chunk& c, const Paths& P, uint2 pk, RGB L) {      
 // at compile time, so the plain kernel keeps its own (smaller) register allocation.
 enum ShadeMode { kPlain, kGuidedMode, kFallbackMode };
 template <int MODE, bool MIX>
-__global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity, bool first) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == kGuidedMode || MIX ? 2 : 3))) k_shade(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity, bool first) {
     constexpr bool GUIDED = MODE == kGuidedMode, FALLBACK = MODE == kFallbackMode;
     const Chunk& c = *cp;
     const uint32_t* in = parity ? q.active1 : q.active0;
     uint32_t* out = q.bin_rays ? q.unsorted : (parity ? q.active0 : q.active1);
     uint32_t* n_out = &q.counts[parity ^ 1];
     const uint32_t n = q.counts[parity];
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t blk = blockIdx.x * blockDim.x; blk < n; blk += stride) {
+    // The block takes its entries a window at a time and orders them by what they hit, so a wave shades one
+    // kind of surface (or none) instead of every kind its lanes met.  Windows of 1,024 entries when they keep
+    // the grid busy, else one round of the block.  (Lanes in use per issued vector instruction 0.40 to 0.66,
+    // vector instructions 38% fewer, 17.7 to 15.4 ms on the 1024x1024 frame of the 2.2M-triangle scene; what
+    // is left is the chain of dependent loads from queue entry to shading data at three waves per SIMD.)
+    constexpr uint32_t kWindow = 1024, kClasses = 16;
+    __shared__ uint32_t s_entry[kWindow];
+    __shared__ uint32_t s_class[kClasses];
+    const uint32_t window = n >= gridDim.x * kWindow ? kWindow : 256u;
+    for (uint32_t blk0 = blockIdx.x * window, blk = 0; blk0 < n;) {
+        const uint32_t m = min(window, n - blk0);
+        if (blk == 0) {
+            if (threadIdx.x < kClasses) s_class[threadIdx.x] = 0u;
+            __syncthreads();
+            uint32_t entry[kWindow / 256], cls[kWindow / 256];
+#pragma unroll
+            for (uint32_t r = 0; r < kWindow / 256; r++) {
+                const uint32_t j = r * 256u + threadIdx.x;
+                cls[r] = kClasses;
+                if (j < m) {
+                    entry[r] = in[blk0 + j];
+                    const int ob = P.hit_ot[FALLBACK ? entry[r] & ~kResumed : entry[r]].x;
+                    cls[r] = 0u;                                            // missed the scene
+                    if (ob >= 0) {
+                        const int4 info = s.obj_info[ob];
+                        cls[r] = info.y >= 0 ? 1u : min(2u + (uint32_t)s.materials[info.x].type, kClasses - 1u);
+                    }
+                    atomicAdd(&s_class[cls[r]], 1u);
+                }
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                uint32_t at = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < kClasses; k++) {
+                    const uint32_t count = s_class[k];
+                    s_class[k] = at;
+                    at += count;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t r = 0; r < kWindow / 256; r++)
+                if (cls[r] < kClasses) s_entry[atomicAdd(&s_class[cls[r]], 1u)] = entry[r];
+            __syncthreads();
+        }
         const uint32_t i = blk + threadIdx.x;
-        bool valid = i < n;
+        bool valid = i < m;
         if (FALLBACK && c.deep == 1) {
             // Park a path that goes on and may draw more values than its sample tables hold (three 1D and
             // three 2D values of the vertex, a roulette value before and after it).
             bool park = false;
             if (valid) {
-                const uint32_t slot = in[i], st = first ? 0u : P.state[slot];
+                const uint32_t slot = s_entry[i], st = first ? 0u : P.state[slot];
                 const int c1 = (int)((st >> 8) & 0xffu), c2 = (int)((st >> 16) & 0xffu), ob = P.hit_ot[slot].x;
                 park = (c1 + (st & kDelta ? 5 : 4) > c.d1 || c2 + 3 > c.d2) && ob >= 0 && s.obj_info[ob].y < 0;
                 if (park) {
@@ -795,7 +839,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restri
         RGB sh_c = rgb(0, 0, 0), mi_f = rgb(0, 0, 0);
         int mi_light = 0;
         if (valid) {
-            slot = FALLBACK ? in[i] & ~kResumed : in[i];
+            slot = FALLBACK ? s_entry[i] & ~kResumed : s_entry[i];
             // the radiance is read where the vertex emits or the path ends, and written back when it changed;
             // with the direct light kept per shadow ray instead of in two zeroed halves per path, and nothing
             // initialised by ray generation, a path moves about 150 bytes less per vertex (k_resolve 1.9 to
@@ -1342,6 +1386,12 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, const Chunk* __restri
                 gi[0] = g_x0; gi[1] = g_x1; gi[2] = g_x2; gi[3] = g_x3;
             }
         }
+        blk += 256u;
+        if (blk >= m) {
+            blk = 0;
+            blk0 += gridDim.x * window;
+            __syncthreads();                                    // the window's entries are read
+        }
     }
 }
 
@@ -1678,6 +1728,7 @@ __global__ void k_film_spill(const Chunk* __restrict__ cp, Paths P, FilmParams f
     const PixelSampler ps = pixel_sampler(c, p);
     const TileBox t = tile_of(v, f.tile_first, px.x, px.y);
     uint32_t bits = 0;
+    int k_first = 0x7fffffff, k_last = -1;              // samples that reach a neighbour lie in this range
     const int ka = c.guided ? c.k0 : 0, kb = c.guided ? min(c.k1, v.spp) : v.spp;
     ImageSamples is(ps, c.jt, ka);
     for (int k = ka; k < kb; k++) {
@@ -1691,7 +1742,11 @@ __global__ void k_film_spill(const Chunk* __restrict__ cp, Paths P, FilmParams f
                 if (xx == px.x && yy == px.y) continue;
                 if (xx < t.px0 || xx >= t.px1 || yy < t.py0 || yy >= t.py1) continue;   // outside Film_Tile
                 if (xx < t.sx0 || xx >= t.sx1 || yy < t.sy0 || yy >= t.sy1) margin = true;
-                else bits |= 1u << ((yy - px.y + 1) * 3 + (xx - px.x + 1));
+                else {
+                    bits |= 1u << ((yy - px.y + 1) * 3 + (xx - px.x + 1));
+                    k_first = min(k_first, k);
+                    k_last = k;
+                }
             }
         if (margin) {
             const uint32_t e = atomicAdd(&q.counts[5], 1u);
@@ -1704,6 +1759,7 @@ __global__ void k_film_spill(const Chunk* __restrict__ cp, Paths P, FilmParams f
         }
     }
     f.spill[p] = (uint8_t)(bits & 0x0fu) | (uint8_t)((bits >> 1) & 0xf0u);   // 9 bits minus the centre
+    if (bits) f.spill_range[p] = make_int2(k_first, k_last);
 }
 
 YG_INLINE bool spill_bit(uint8_t packed, int dx, int dy) {       // direction from source to target
@@ -1718,6 +1774,10 @@ YG_INLINE void gather(const Chunk& c, const Paths& P, const FilmParams& f, const
     if (nx < t.sx0 || nx >= t.sx1 || ny < t.sy0 || ny >= t.sy1) return;
     const long long li = t.first + (long long)(ny - t.sy0) * (t.sx1 - t.sx0) + (nx - t.sx0) - f.base;   // chunk-local
     if (!spill_bit(f.spill[li], x - nx, y - ny)) return;
+    // almost always one sample: going through all of the neighbour's cost 0.8 of 0.86 ms at 1,024 spp
+    const int2 range = f.spill_range[li];
+    ka = max(ka, range.x);
+    kb = min(kb, range.y + 1);
     ImageSamples is(pixel_sampler(c, (int)li), c.jt, ka);
     for (int k = ka; k < kb; k++) {
         float jx, jy;
