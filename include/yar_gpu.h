@@ -348,10 +348,11 @@ int  yar_gpu_trace_rays_device(yar_gpu_ctx* ctx, const yar_ray* d_rays, int64_t 
                                yar_hit* d_hits, void* hip_stream);
 /* Allocation-free form of yar_gpu_trace_rays_device.  No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  It calls no allocating routine; the per-ray hit staging and the traversal
- * counters live in a static device array of 24 MB (each device the library runs on holds its own copy
- * until the process ends), so count must not exceed 2^20 rays (YAR_ERR_CAPACITY otherwise).  Every
- * call on one device shares that array: calls that overlap on one device race. */
+ * forbid hipMalloc).  It calls no allocating routine; the work cursors, the traversal counters and the
+ * hits of calls whose rays and hits share memory live in a static device array of 24 MB (each device
+ * the library runs on holds its own copy until the process ends), so count must not exceed 2^20 rays
+ * (YAR_ERR_CAPACITY otherwise).  Every call on one device shares that array: calls that overlap on one
+ * device race. */
 int  yar_gpu_trace_rays_device_noalloc(yar_gpu_ctx* ctx, const yar_ray* d_rays, int64_t count, int32_t any_hit,
                                        yar_hit* d_hits, void* hip_stream);
 /* Per-ray traversal counters of the last trace_rays call (requires enable_counters). */

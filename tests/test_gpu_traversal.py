@@ -2,6 +2,7 @@
 are one leaf, stacks that overflow, queues shorter and longer than one batch per wave."""
 import numpy as np
 import pytest
+import torch
 
 import yar_amd
 from tests import raygen
@@ -163,3 +164,32 @@ def test_short_and_long_runs_in_one_batch(c1_path):
         ctx.set_views([v])
         img, _, rvar, _ = ctx.render(0, want_film=False)
         assert np.array_equal(img, imgs[i]) and rvar == var[i]
+
+
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 5119, 327679, 327681, 700001])
+def test_ray_batches_of_every_length(count, c1_path):
+    """A batch is answered ray by ray whatever its length: lengths around one wave, one ray per wave, the
+    rays all waves take first (320K) and several runs per wave, as prefixes of one batch."""
+    scene = yar_amd.Scene(c1_path)
+    ctx = yar_amd.Context(scene)
+    rays = raygen.random_rays(scene, 700001, seed=29)
+    rays["tmax"] = np.where(np.arange(rays.size) % 3 == 0, 1.0, np.inf).astype(np.float32)
+    for any_hit in (False, True):
+        whole = np.concatenate([ctx.trace_rays(rays[i:i + 100000], any_hit=any_hit) for i in range(0, rays.size, 100000)])
+        got = ctx.trace_rays(rays[:count], any_hit=any_hit)
+        assert got.tobytes() == whole[:count].tobytes()
+
+
+@pytest.mark.parametrize("count", [64, 400001])
+def test_device_rays_and_hits_in_one_buffer(count, c1_path):
+    """Hits written over the rays they answer: every ray is read before."""
+    scene = yar_amd.Scene(c1_path)
+    ctx = yar_amd.Context(scene)
+    rays = raygen.random_rays(scene, count, seed=31)
+    want = ctx.trace_rays(rays).tobytes()
+    for entry in (ctx.trace_rays_device, ctx.trace_rays_device_noalloc):
+        buf = torch.from_numpy(rays.view(np.uint8).reshape(-1).copy()).cuda()
+        torch.cuda.synchronize()
+        entry(buf.data_ptr(), count, buf.data_ptr())
+        torch.cuda.synchronize()
+        assert buf[:24 * count].cpu().numpy().tobytes() == want

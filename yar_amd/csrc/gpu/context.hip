@@ -158,16 +158,19 @@ struct KernelTimer {
     ~KernelTimer() { for (auto e : pool) (void)hipEventDestroy(e); }
 };
 
-// Scratch of the allocation-free ray queries (yar_gpu_trace_rays_device_noalloc): per-ray hit staging
-// (t and barycentrics, object and triangle) for up to kNoAllocMaxRays rays, then the 16 traversal
-// counters.  Each device holds its own copy from module load until the process ends, and every call
-// on a device shares it.  In host code `scratch` names no device address: kernels receive the address
+// Scratch of the allocation-free ray queries (yar_gpu_trace_rays_device_noalloc): the traversal counters
+// and the work cursors, then hit staging for calls whose rays and hits share memory.  Each device holds its own copy from module load until the process ends, and every
+// call on a device shares it.  In host code `scratch` names no device address: kernels receive the address
 // hipGetSymbolAddress returned for the current device (scratch_ptr below).
 constexpr int64_t kNoAllocMaxRays = (int64_t)1 << 20;
-constexpr size_t kNoAllocTbBytes = (size_t)kNoAllocMaxRays * sizeof(float4);
-constexpr size_t kNoAllocOtBytes = (size_t)kNoAllocMaxRays * sizeof(int2);
-constexpr size_t kNoAllocScratchBytes = kNoAllocTbBytes + kNoAllocOtBytes + 16 * sizeof(unsigned long long);
-__device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+constexpr size_t kNoAllocWordBytes = (size_t)kRayWords * sizeof(uint32_t);
+__device__ __align__(256) unsigned char scratch[kNoAllocWordBytes + (size_t)kNoAllocMaxRays * sizeof(yar_hit)];
+
+// Whether the two arrays of a device ray query share memory: every ray is then read before a hit is written.
+bool overlapping(const yar_ray* rays, const yar_hit* hits, int64_t count) {
+    const uintptr_t r = (uintptr_t)rays, h = (uintptr_t)hits;
+    return r < h + (size_t)count * sizeof(yar_hit) && h < r + (size_t)count * sizeof(yar_ray);
+}
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -186,16 +189,13 @@ unsigned char* scratch_ptr(int device) {
     return g_scratch_ptr[device];
 }
 
-__global__ void k_zero_u64(unsigned long long* p, int n) {
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
-}
-
 }  // namespace
 
 struct yar_gpu_ctx {
     std::string error;
     int device = 0;
     int cu_count = 1;
+    int ray_grid = 1;                     // blocks of the persistent ray-query kernel
     unsigned char* scratch = nullptr;     // this device's address of the allocation-free scratch array
     hipStream_t stream = nullptr;
     yar_gpu_options opt{};
@@ -264,8 +264,9 @@ struct yar_gpu_ctx {
     Paths graph_P{};
     Queues graph_q{};
     // trace_rays buffers
-    DevBuf<float4> tr_rays, tr_tb;
-    DevBuf<int2> tr_ot;
+    DevBuf<float4> tr_rays;
+    DevBuf<yar_hit> tr_hits;
+    DevBuf<unsigned long long> tr_words;  // counters and work cursors
     yar_render_stats last_trace{};
 
     void drop_graph() {
@@ -282,7 +283,7 @@ struct yar_gpu_ctx {
         objs.release();
         DevBuf<float4>* b4[] = {&tri_verts, &obj_o2w, &obj_nrm, &vtx_n, &ray_o, &ray_d, &coeff, &L, &dl_coeff,
                                 &dl_bsdf, &hit_tb, &radiance, &sh_o, &sh_d, &sh_c, &mi_o, &mi_d,
-                                &mi_f, &out_film, &side_rad, &tr_rays, &tr_tb};
+                                &mi_f, &out_film, &side_rad, &tr_rays};
         for (auto* b : b4) b->release();
         DevBuf<int4>* bi4[] = {&obj_info, &mesh_info, &tri_vidx, &side_info};
         for (auto* b : bi4) b->release();
@@ -291,7 +292,7 @@ struct yar_gpu_ctx {
         vtx_uv.release(); materials.release(); rects.release(); points.release();
         spots.release(); dirs.release(); mesh_lights.release(); mesh_light_cdf.release(); spheres.release(); env.release();
         pixels.release(); pix_first.release(); dviews.release(); chunks.release(); chunk_slot.release();
-        perm.release(); jump_lo.release(); jump_hi.release(); hit_ot.release(); tr_ot.release(); state.release(); rng.release();
+        perm.release(); jump_lo.release(); jump_hi.release(); hit_ot.release(); tr_hits.release(); tr_words.release(); state.release(); rng.release();
         DevBuf<uint32_t>* bu[] = {&q_a, &q_b, &mi_path, &dl_path, &dl_shadow, &counts, &q_unsorted};
         sh_seen.release();
         for (auto* b : bu) b->release();
@@ -1018,7 +1019,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     ctx->sh_seen.reserve(np);
     for (auto* b : qb) b->reserve(np);
     ctx->mi_ndw.reserve(np);
-    ctx->counts.reserve(16);
+    ctx->counts.reserve(counter(kCounters + 3 * kSlices));
     const int bin_mode = std::min(std::max(ctx->opt.bin_rays, 0), 3);
     const bool bin_rays = bin_mode > 0;
     if (bin_rays) {
@@ -1154,7 +1155,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         }
     }
     ctx->chunks.upload(hc, s);
-    HIPX(hipMemsetAsync(ctx->counts.p, 0, 16 * sizeof(uint32_t), s));
+    HIPX(hipMemsetAsync(ctx->counts.p, 0, counter(kCounters + 3 * kSlices) * sizeof(uint32_t), s));
     HIPX(hipMemsetAsync(ctx->totals.p, 0, 24 * sizeof(unsigned long long), s));
 
     Paths P{};
@@ -1209,9 +1210,9 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     const bool use_graph = ctx->opt.use_graph != 0 && !guided;
     Chunk* slot = ctx->chunk_slot.p;
 
-    // polling slots: a ring of four times 16 counters for the iterations, one per (chunk, pass) completion check (graph) and
+    // polling slots: a ring of four times the counters for the iterations, one per (chunk, pass) completion check (graph) and
     // one for the training-record count
-    const size_t poll_n = 64 + hc.size() + 1;
+    const size_t poll_ring = 4 * counter(kCounters), poll_n = poll_ring + hc.size() + 1;
     if (ctx->h_poll_n < poll_n) {
         if (ctx->h_poll) (void)hipHostFree(ctx->h_poll);
         ctx->h_poll = nullptr;
@@ -1258,8 +1259,9 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
     auto run_iterations = [&](int64_t limit, bool fresh) {
         constexpr int kRing = 4;                     // polling slots and events in use at a time: three
         auto idle = [&](int64_t it) {
-            const uint32_t* c = hp + (it % kRing) * 16;
-            return c[(it & 1) ^ 1] == 0 && c[light_count_base((int)(it & 1)) + 2] == 0;
+            const uint32_t* c = hp + (it % kRing) * counter(kCounters);
+            const int parity = (int)(it & 1);
+            return c[counter(parity ^ 1)] == 0 && c[counter(light_count_base(parity) + 2)] == 0;
         };
         int64_t it = 0;
         for (; it < limit; it++) {
@@ -1278,7 +1280,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
             } else {
                 launch_iteration(ctx->scene, slot, P, q, parity, fresh && it == 0, lc);
             }
-            HIPX(hipMemcpyAsync(hp + (it % kRing) * 16, ctx->counts.p, 16 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipMemcpyAsync(hp + (it % kRing) * counter(kCounters), ctx->counts.p, counter(kCounters) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             HIPX(hipEventRecord(ev[it % kRing], s));
         }
         HIPX(hipEventSynchronize(ev[(it - 1) % kRing]));
@@ -1289,7 +1291,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         if (use_graph) {
             HIPX(hipGraphLaunch(ctx->graph, s));
             // the active list the last iteration wrote must be empty
-            HIPX(hipMemcpyAsync(hp + 64 + sp.hc, ctx->counts.p + (iters & 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipMemcpyAsync(hp + poll_ring + sp.hc, ctx->counts.p + counter(iters & 1), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         } else {
             kt.begin(4);
             launch_raygen(slot, c.n_paths, P, q, s);
@@ -1337,7 +1339,7 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         if (last_of_chunk) run_film(sp);
         if (guided && (si + 1 == steps.size() || steps[si + 1].pass != sp.pass)) {
             // end of a guided pass: train the proposal on the records it produced
-            HIPX(hipMemcpyAsync(hp + poll_n - 1, ctx->counts.p + 10, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+            HIPX(hipMemcpyAsync(hp + poll_n - 1, ctx->counts.p + counter(10), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             HIPX(hipStreamSynchronize(s));
             const int64_t n_rec = std::min<int64_t>(hp[poll_n - 1], train_cap);
             train_records = hp[poll_n - 1];
@@ -1358,18 +1360,18 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
         HIPX(hipMemcpyAsync(ctx->h_var.p, ctx->out_var.p, total_pixels * sizeof(double), hipMemcpyDeviceToHost, s));
     }
     unsigned long long tot[24];
-    uint32_t cnt[16];
+    std::vector<uint32_t> cnt((size_t)counter(kCounters));
     HIPX(hipMemcpyAsync(tot, ctx->totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
-    HIPX(hipMemcpyAsync(cnt, ctx->counts.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
+    HIPX(hipMemcpyAsync(cnt.data(), ctx->counts.p, cnt.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     HIPX(hipStreamSynchronize(s));
     for (auto e : ev) (void)hipEventDestroy(e);
     if (use_graph)
         for (const Step& sp : steps)
-            if (hp[64 + sp.hc] != 0) loop_ok = false;
+            if (hp[poll_ring + sp.hc] != 0) loop_ok = false;
     if (!loop_ok) throw HipError{"bounce loop did not terminate within max_light_bounces + 2 iterations"};
     double ksec[kTimerKinds];
     kt.collect(ksec);
-    const uint32_t n_side = cnt[5];
+    const uint32_t n_side = cnt[counter(5)];
     if ((int64_t)n_side > side_cap) throw HipError{"film side list overflow", YAR_ERR_CAPACITY};
     std::vector<float4> side_rad(n_side);
     std::vector<int4> side_info(n_side);
@@ -1616,6 +1618,7 @@ int yar_gpu_create(const yar_scene_desc* scene, const yar_gpu_options* options, 
         ctx->scratch = scratch_ptr(ctx->device);
         upload_scene(ctx.get(), scene);
         upload_jump_tables(ctx.get());
+        ctx->ray_grid = ctx->cu_count * trace_rays_blocks_per_cu(ctx->launch_cfg());
         yar_view v{};
         std::memcpy(v.camera_to_world, scene->camera.camera_to_world, sizeof(v.camera_to_world));
         v.fov_y_degrees = scene->camera.fov_y_degrees;
@@ -1841,28 +1844,17 @@ int yar_gpu_trace_rays(yar_gpu_ctx* ctx, const yar_ray* rays, int64_t count, int
         HIPX(hipSetDevice(ctx->device));
         hipStream_t s = ctx->stream;
         ctx->tr_rays.reserve(2 * (size_t)count);
-        ctx->tr_tb.reserve((size_t)count);
-        ctx->tr_ot.reserve((size_t)count);
-        ctx->totals.reserve(16);
+        ctx->tr_hits.reserve((size_t)count);
+        ctx->tr_words.reserve(kRayWords / 2);
         HIPX(hipMemcpyAsync(ctx->tr_rays.p, rays, (size_t)count * sizeof(yar_ray), hipMemcpyHostToDevice, s));
-        HIPX(hipMemsetAsync(ctx->totals.p, 0, 16 * sizeof(unsigned long long), s));
         LaunchCfg lc = ctx->launch_cfg();
-        launch_trace_rays(ctx->scene, ctx->tr_rays.p, count, any_hit, ctx->tr_tb.p, ctx->tr_ot.p, ctx->totals.p, lc);
+        lc.trav_grid = ctx->ray_grid;
+        launch_trace_rays(ctx->scene, ctx->tr_rays.p, count, any_hit, ctx->tr_hits.p, ctx->tr_words.p, lc);
         HIPX(hipGetLastError());
-        std::vector<float4> tb(count);
-        std::vector<int2> ot(count);
-        unsigned long long tot[16];
-        HIPX(hipMemcpyAsync(tb.data(), ctx->tr_tb.p, (size_t)count * sizeof(float4), hipMemcpyDeviceToHost, s));
-        HIPX(hipMemcpyAsync(ot.data(), ctx->tr_ot.p, (size_t)count * sizeof(int2), hipMemcpyDeviceToHost, s));
-        HIPX(hipMemcpyAsync(tot, ctx->totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
+        unsigned long long tot[16] = {};
+        HIPX(hipMemcpyAsync(out_hits, ctx->tr_hits.p, (size_t)count * sizeof(yar_hit), hipMemcpyDeviceToHost, s));
+        if (lc.counters) HIPX(hipMemcpyAsync(tot, ctx->tr_words.p, sizeof(tot), hipMemcpyDeviceToHost, s));
         HIPX(hipStreamSynchronize(s));
-        for (int64_t i = 0; i < count; i++) {
-            yar_hit& h = out_hits[i];
-            h.t = tb[i].x;
-            h.object = ot[i].x;
-            h.triangle = ot[i].y;
-            h.barycentrics[0] = tb[i].y; h.barycentrics[1] = tb[i].z; h.barycentrics[2] = tb[i].w;
-        }
         ctx->last_trace = yar_render_stats{};
         ctx->last_trace.node_visits = (int64_t)tot[12];
         ctx->last_trace.leaf_refs = (int64_t)tot[13];
@@ -1874,19 +1866,6 @@ int yar_gpu_trace_rays(yar_gpu_ctx* ctx, const yar_ray* rays, int64_t count, int
 
 }  // extern "C"
 
-namespace {
-__global__ void k_pack_hits(const float4* __restrict__ tb, const int2* __restrict__ ot, long long n, yar_hit* out) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float4 a = tb[i];
-    int2 b = ot[i];
-    yar_hit h;
-    h.t = a.x; h.object = b.x; h.triangle = b.y;
-    h.barycentrics[0] = a.y; h.barycentrics[1] = a.z; h.barycentrics[2] = a.w;
-    out[i] = h;
-}
-}  // namespace
-
 extern "C" int yar_gpu_trace_rays_device(yar_gpu_ctx* ctx, const yar_ray* d_rays, int64_t count, int32_t any_hit,
                                          yar_hit* d_hits, void* hip_stream) {
     if (!ctx || count < 0 || (count > 0 && (!d_rays || !d_hits)))
@@ -1894,17 +1873,17 @@ extern "C" int yar_gpu_trace_rays_device(yar_gpu_ctx* ctx, const yar_ray* d_rays
     if (count == 0) return YAR_OK;
     return guarded(ctx, "yar_gpu_trace_rays_device", [&] {
         HIPX(hipSetDevice(ctx->device));
-        ctx->tr_tb.reserve((size_t)count);
-        ctx->tr_ot.reserve((size_t)count);
-        ctx->totals.reserve(16);
+        ctx->tr_words.reserve(kRayWords / 2);
         LaunchCfg lc = ctx->launch_cfg();
+        lc.trav_grid = ctx->ray_grid;
         if (hip_stream) lc.stream = (hipStream_t)hip_stream;
-        HIPX(hipMemsetAsync(ctx->totals.p, 0, 16 * sizeof(unsigned long long), lc.stream));
-        launch_trace_rays(ctx->scene, reinterpret_cast<const float4*>(d_rays), count, any_hit, ctx->tr_tb.p, ctx->tr_ot.p,
-                          ctx->totals.p, lc);
-        hipLaunchKernelGGL(k_pack_hits, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, lc.stream, ctx->tr_tb.p,
-                           ctx->tr_ot.p, (long long)count, d_hits);
+        const bool staged = overlapping(d_rays, d_hits, count);
+        if (staged) ctx->tr_hits.reserve((size_t)count);
+        launch_trace_rays(ctx->scene, reinterpret_cast<const float4*>(d_rays), count, any_hit, staged ? ctx->tr_hits.p : d_hits,
+                          ctx->tr_words.p, lc);
         HIPX(hipGetLastError());
+        if (staged)
+            HIPX(hipMemcpyAsync(d_hits, ctx->tr_hits.p, (size_t)count * sizeof(yar_hit), hipMemcpyDeviceToDevice, lc.stream));
     });
 }
 
@@ -1920,9 +1899,9 @@ extern "C" int yar_gpu_get_info(const yar_gpu_ctx* ctx, yar_gpu_info* out_info) 
     return YAR_OK;
 }
 
-// Allocation-free form of yar_gpu_trace_rays_device: the same kernels, with the hit staging and the
-// counters in this device's `scratch` array instead of context buffers, cleared by a kernel (no
-// memset node), so the call can sit inside a HIP graph capture or a loop that must not allocate.
+// Allocation-free form of yar_gpu_trace_rays_device: the same kernel, with the counters in this device's
+// `scratch` array instead of a context buffer, cleared by a kernel (no memset node), so the call can sit
+// inside a HIP graph capture or a loop that must not allocate.
 extern "C" int yar_gpu_trace_rays_device_noalloc(yar_gpu_ctx* ctx, const yar_ray* d_rays, int64_t count, int32_t any_hit,
                                                  yar_hit* d_hits, void* hip_stream) {
     if (!ctx || count < 0 || (count > 0 && (!d_rays || !d_hits)))
@@ -1933,15 +1912,14 @@ extern "C" int yar_gpu_trace_rays_device_noalloc(yar_gpu_ctx* ctx, const yar_ray
     return guarded(ctx, "yar_gpu_trace_rays_device_noalloc", [&] {
         HIPX(hipSetDevice(ctx->device));
         if (!ctx->scratch) throw HipError{"scratch array not set up for this device"};
-        float4* tb = reinterpret_cast<float4*>(ctx->scratch);
-        int2* ot = reinterpret_cast<int2*>(ctx->scratch + kNoAllocTbBytes);
-        unsigned long long* totals = reinterpret_cast<unsigned long long*>(ctx->scratch + kNoAllocTbBytes + kNoAllocOtBytes);
         LaunchCfg lc = ctx->launch_cfg();
+        lc.trav_grid = ctx->ray_grid;
         if (hip_stream) lc.stream = (hipStream_t)hip_stream;
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, lc.stream, totals, 16);
-        launch_trace_rays(ctx->scene, reinterpret_cast<const float4*>(d_rays), count, any_hit, tb, ot, totals, lc);
-        hipLaunchKernelGGL(k_pack_hits, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, lc.stream, tb, ot,
-                           (long long)count, d_hits);
+        const bool staged = overlapping(d_rays, d_hits, count);
+        yar_hit* staging = reinterpret_cast<yar_hit*>(ctx->scratch + kNoAllocWordBytes);
+        launch_trace_rays(ctx->scene, reinterpret_cast<const float4*>(d_rays), count, any_hit, staged ? staging : d_hits,
+                          reinterpret_cast<unsigned long long*>(ctx->scratch), lc);
         HIPX(hipGetLastError());
+        if (staged) HIPX(hipMemcpyAsync(d_hits, staging, (size_t)count * sizeof(yar_hit), hipMemcpyDeviceToDevice, lc.stream));
     });
 }

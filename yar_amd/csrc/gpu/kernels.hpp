@@ -59,9 +59,14 @@ constexpr uint32_t kDlMis = 1u << 31;
 constexpr uint32_t kNoSlot = 0xffffffffu;
 
 // Work queues.  The active path list ping-pongs between two buffers; `parity` selects the input.
-// counts: [0], [1] active lists, [2] shadow, [3] mis, [4] dl of even iterations, [12] [13] [14] of odd
-//         ones, [5] film side entries, [6] [7] [8] work-fetch cursors of the traversal (path rays or all,
-//         shadow rays, MIS rays launched alone), [9] guide queries, [10] training records.
+// counts, each on a cache line of its own (counter(k) is counter k's word): [0], [1] active lists,
+// [2] shadow, [3] mis, [4] dl of even iterations, [12] [13] [14] of odd ones, [5] film side entries,
+// [9] guide queries, [10] training records, [16..39] work cursors of the traversal, one per queue slice
+// (8 for path rays or all, 8 for shadow rays, 8 for MIS rays launched alone).
+// Atomics serialize per line: with all counters on one, every append and every fetch of a launch queued
+// behind each other.
+constexpr int kCounters = 16, kSlices = 8, kCounterWords = 32;
+__host__ __device__ inline int counter(int k) { return k * kCounterWords; }
 __host__ __device__ inline int light_count_base(int parity) { return parity ? 12 : 2; }
 struct Queues {
     uint32_t* active0;
@@ -169,8 +174,11 @@ enum IterStage {
 void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, bool first, const LaunchCfg& cfg);
 void launch_iteration(const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, bool first, const LaunchCfg& cfg);
 void launch_film(const Chunk* c, int n_pixels, const Paths& p, FilmParams f, Queues q, hipStream_t s);
-void launch_trace_rays(const DevScene& sc, const float4* rays, int64_t n, int any, float4* out_tb, int2* out_ot,
-                       unsigned long long* totals, const LaunchCfg& cfg);
+// Ray queries; `totals` holds 16 traversal counters and, in lines of their own behind them, the work cursors of the slices.
+constexpr int kRayWords = kCounterWords * (1 + kSlices);
+void launch_trace_rays(const DevScene& sc, const float4* rays, int64_t n, int any, yar_hit* hits, unsigned long long* totals,
+                       const LaunchCfg& cfg);
+int trace_rays_blocks_per_cu(const LaunchCfg& cfg);
 int traversal_blocks_per_cu(const LaunchCfg& cfg);
 
 }  // namespace yg

@@ -56,14 +56,6 @@ YG_INLINE void block_append(uint32_t* const (&ctr)[NQ], const bool (&pred)[NQ], 
     __syncthreads();
 }
 
-// Next `size` work items (a multiple of 64) for this wave from a device cursor (persistent
-// traversal kernels).
-YG_INLINE uint32_t wave_fetch(uint32_t* cursor, uint32_t size) {
-    uint32_t base = 0;
-    if (__lane_id() == 0) base = atomicAdd(cursor, size);
-    return __shfl(base, 0);
-}
-
 // Traversal counters per kernel kind: totals[4*kind + 0..3] = nodes, leaf refs, triangle tests,
 // objects; kind 0 extend, 1 shadow, 2 mis, 3 trace_rays.
 template <bool COUNT>
@@ -478,10 +470,10 @@ __global__ void k_raygen(const Chunk* __restrict__ cp, Paths P, Queues q) {
     if (c.uniform_spp > 0 && !c.guided && !c.sequential) {
         // every slot below n_paths is a path: the queue is the identity, no appends
         if (active) q.active0[s] = (uint32_t)s;
-        if (s == 0) q.counts[0] = (uint32_t)c.n_paths;
+        if (s == 0) q.counts[counter(0)] = (uint32_t)c.n_paths;
         return;
     }
-    uint32_t* const ctr[1] = {&q.counts[0]};
+    uint32_t* const ctr[1] = {&q.counts[counter(0)]};
     const bool pred[1] = {active};
     uint32_t idx[1];
     block_append<1>(ctr, pred, idx);
@@ -491,11 +483,11 @@ __global__ void k_raygen(const Chunk* __restrict__ cp, Paths P, Queues q) {
 // Clears the queue counters and cursors before a pass; the film side-list counter [5] and the
 // training-record counter [10] run on.
 __global__ void k_zero_counts(uint32_t* counts, int n) {
-    if ((int)threadIdx.x < n && threadIdx.x != 5 && threadIdx.x != 10) counts[threadIdx.x] = 0u;
+    if ((int)threadIdx.x < n && threadIdx.x != 5 && threadIdx.x != 10) counts[counter(threadIdx.x)] = 0u;
 }
 
 void launch_raygen(const Chunk* c, long long n_paths_max, const Paths& p, Queues q, hipStream_t s) {
-    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, q.counts, 16);
+    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, q.counts, kCounters);
     hipLaunchKernelGGL(k_raygen, dim3((unsigned)((n_paths_max + 255) / 256)), dim3(256), 0, s, c, p, q);
 }
 
@@ -517,7 +509,7 @@ __global__ void k_resume(const Chunk* __restrict__ cp, Paths P, Queues q) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t slot = kNoSlot;
     if (p < c.n_pixels && P.first_parked[p] != 0x7fffffff) slot = take_parked(c, P, p, P.first_parked[p]);
-    uint32_t* const ctr[1] = {&q.counts[0]};
+    uint32_t* const ctr[1] = {&q.counts[counter(0)]};
     const bool pred[1] = {slot != kNoSlot};
     uint32_t idx[1];
     block_append<1>(ctr, pred, idx);
@@ -525,7 +517,7 @@ __global__ void k_resume(const Chunk* __restrict__ cp, Paths P, Queues q) {
 }
 
 void launch_resume(const Chunk* c, int n_pixels, const Paths& p, Queues q, hipStream_t s) {
-    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, q.counts, 16);
+    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, s, q.counts, kCounters);
     hipLaunchKernelGGL(k_resume, dim3((n_pixels + 255) / 256), dim3(256), 0, s, c, p, q);
 }
 
@@ -550,30 +542,81 @@ YG_INLINE void with_stacks(StackCfg cfg, Body body) {
     }
 }
 
-// Persistent traversal over a device queue.  A wave takes runs of `size` entries: the first one is its by
-// position (no atomic, so a launch over a short queue costs almost nothing), the others come from the
-// cursor, 256 entries at a time while more than 8 fetches per wave remain (fewer same-address atomics),
-// then 64 (balanced tail).  A lane whose query ended takes the run's next entry once cfg.refill lanes of
-// its wave are idle, so a wave is not held by its longest ray (24 idle lanes against 64, i.e. whole
-// batches: 84 against 103 ms on the 1024x1024 frame of the 2.2M-triangle scene, 8 and 32 within 1%).
-// A queue of less than a batch per wave is spread over all waves: one ray's chain of dependent loads and
-// branches is what such a launch lasts, and in a wave of its own a ray does not wait for 63 others
-// (64x64 tile at 4 spp: 2.7 to 1.7 ms per render).
+// Persistent traversal over a device queue.  A queue of 64 entries per wave or more is cut into kSlices
+// slices, and the blocks of an XCD (dealt round-robin) start on one of them.  A wave takes runs of entries:
+// the first one is its by position, the others come from its slice's cursor, 256 entries at a time while
+// more than 8 such fetches per wave remain, then 64 (balanced tail), and from the other slices once its own
+// is done.  One cursor per slice, on a line of its own, because atomics on one address serialize; and the
+// ticket of the run behind the current one is drawn when the current one is begun, so its 1 to 2 us pass
+// while the wave traces.  Within the last kAhead entries per wave no ticket is drawn ahead: a wave busy with
+// long rays would hold a run that idle waves could take.  (One cursor, fetched when needed:
+// seven 512x512 views of a small room in one batch 16.2 ms, 1024x1024 at 64 spp of the 2.2M-triangle scene
+// 67.7; so 14.6 and 65.5.  Eight cursors, looked at before each draw and none drawn early: 16.8 and 75.)
+// A lane whose query ended takes the run's next entry once cfg.refill lanes of its wave are idle, so a wave
+// is not held by its longest ray (24 idle lanes against 64, i.e. whole batches: 84 against 103 ms on the
+// 1024x1024 frame of the 2.2M-triangle scene, 8 and 32 within 1%).
+// A queue of less than a batch per wave is spread over all waves, without cursors: one ray's chain of
+// dependent loads and branches is what such a launch lasts, and in a wave of its own a ray does not wait for
+// 63 others (64x64 tile at 4 spp: 2.7 to 1.7 ms per render).  It is not cut into slices: path, shadow and MIS
+// rays would lie on XCDs of their own, of unequal length (0.92 to 0.96 ms per render).
 // setup(index, o, d, tmax, any) returns the payload finish(payload, tracer) receives.
+constexpr uint32_t kNoTicket = 0xffffffffu, kAhead = 6u * 64u;
+YG_INLINE bool long_runs(uint32_t n, uint32_t waves) { return n > 8u * 256u * waves; }
 template <bool COUNT, class Stack, class Setup, class Finish>
 YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Stack& st, int depth, TravCounters& cnt,
                            StackCfg cfg, Setup setup, Finish finish) {
     Tracer<COUNT> tr;
     tr.phase = tr.kDone;
     const uint32_t wpb = (blockDim.x + 63u) >> 6;
-    const uint32_t waves = gridDim.x * wpb;
-    uint32_t size = n > 8u * 256u * waves ? 256u : 64u;
-    if (n < 64u * waves) size = max(1u, (n + waves - 1u) / waves);
-    const uint32_t static_end = waves * size;
     const uint32_t lane = __lane_id();
-    uint32_t next = __builtin_amdgcn_readfirstlane((blockIdx.x * wpb + (threadIdx.x >> 6)) * size);
-    uint32_t end = min(next + size, n);
-    bool more = static_end < n;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool spread = n < 64u * gridDim.x * wpb;
+    uint32_t size, slice = 0u, slices_left = 0u, next, end;
+    uint32_t ticket = kNoTicket;        // in lane 0
+    // first entry of slice s's cursor, first entry behind the slice, and the entries one run per wave takes
+    auto bounds = [&](uint32_t n, uint32_t s, uint32_t run, uint32_t& base, uint32_t& stop, uint32_t& round) {
+        const uint32_t part = (n + kSlices - 1u) / kSlices;
+        round = gridDim.x > s ? (gridDim.x - s + kSlices - 1u) / kSlices * wpb * run : 0u;
+        stop = min((s + 1u) * part, n);
+        base = min(s * part, n) + round;
+    };
+    if (spread) {
+        size = max(1u, (n + gridDim.x * wpb - 1u) / (gridDim.x * wpb));
+        next = min((blockIdx.x * wpb + wave) * size, n);
+        end = min(next + size, n);
+    } else {
+        size = long_runs(n, gridDim.x * wpb) ? 256u : 64u;
+        slice = blockIdx.x % kSlices;
+        slices_left = kSlices;
+        uint32_t base, stop, round;
+        bounds(n, slice, size, base, stop, round);
+        next = min(base - round + (blockIdx.x / kSlices * wpb + wave) * size, stop);
+        end = min(next + size, stop);
+        if (base < stop && stop - base > kAhead / size * round && lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, size);
+    }
+    // the next run of the wave's slice, or of the first one behind it that is not used up
+    auto fetch = [&]() {
+        uint32_t m = n;
+        asm volatile("" : "+s"(m));     // computed again here, not kept in registers the traversal needs
+        const uint32_t run = long_runs(m, gridDim.x * wpb) ? 256u : 64u;
+        for (; slices_left > 0u; slices_left--, slice = (slice + 1u) % kSlices) {
+            uint32_t base, stop, round;
+            bounds(m, slice, run, base, stop, round);
+            if (base >= stop) continue;
+            uint32_t at = __builtin_amdgcn_readfirstlane(ticket);
+            if (at == kNoTicket) {
+                if (lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, size);
+                at = __builtin_amdgcn_readfirstlane(ticket);
+            }
+            ticket = kNoTicket;
+            if (at >= stop - base) continue;
+            next = base + at;
+            end = min(next + size, stop);
+            if (size > 64u && !long_runs((stop - end) * kSlices, gridDim.x * wpb)) size = 64u;
+            if (stop - end > kAhead / run * round && lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, size);
+            return;
+        }
+    };
     bool has = false;
     uint32_t payload = 0;
     for (uint32_t turn = 0; turn < kMaxTurns; turn++) {
@@ -581,12 +624,7 @@ YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Sta
         const int n_idle = __builtin_amdgcn_readfirstlane((int)__popcll(idle));
         if (n_idle >= cfg.refill) {
             if (tr.phase == tr.kDone && has) { finish(payload, tr); has = false; }
-            if (next >= end && more) {
-                next = __builtin_amdgcn_readfirstlane(static_end + wave_fetch(cursor, size));
-                end = min(next + size, n);
-                more = next < n;
-                if (size == 256u && n - min(end, n) < 8u * 256u * waves) size = 64u;
-            }
+            if (next >= end && slices_left > 0) fetch();
             if (next < end) {
                 const uint32_t i = next + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
                 if (tr.phase == tr.kDone && i < end) {
@@ -666,9 +704,9 @@ constexpr uint32_t kKindShift = 30, kPathRay = 0u << kKindShift, kShadowRay = 1u
 template <bool COUNT, bool PRIV>
 __global__ void YG_TRAV_BOUNDS k_trace(DevScene sc, Paths P, Queues q, int parity, int kinds, StackCfg cfg) {
     const uint32_t* in = parity ? q.active1 : q.active0;
-    const uint32_t* light_counts = q.counts + light_count_base(parity ^ 1);
-    const uint32_t n_path = kinds & 1 ? q.counts[parity] : 0u, n_shadow = kinds & 2 ? light_counts[0] : 0u,
-                   n_mis = kinds & 4 ? light_counts[1] : 0u;
+    const uint32_t* light_counts = q.counts + counter(light_count_base(parity ^ 1));
+    const uint32_t n_path = kinds & 1 ? q.counts[counter(parity)] : 0u, n_shadow = kinds & 2 ? light_counts[counter(0)] : 0u,
+                   n_mis = kinds & 4 ? light_counts[counter(1)] : 0u;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (kinds & 1) {
             atomicAdd(&q.totals[16], (unsigned long long)n_path);
@@ -679,7 +717,7 @@ __global__ void YG_TRAV_BOUNDS k_trace(DevScene sc, Paths P, Queues q, int parit
     }
     TravCounters cnt = {0, 0, 0, 0};
     with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
-        trace_queue<COUNT>(sc, n_path + n_shadow + n_mis, &q.counts[kinds & 1 ? 6 : kinds & 2 ? 7 : 8], st, depth, cnt, cfg,
+        trace_queue<COUNT>(sc, n_path + n_shadow + n_mis, &q.counts[counter(kCounters + kSlices * (kinds & 1 ? 0 : kinds & 2 ? 1 : 2))], st, depth, cnt, cfg,
             [&](uint32_t i, V3& o, V3& d, float& tmax, bool& any) -> uint32_t {
                 any = false;
                 tmax = f_inf();
@@ -736,7 +774,7 @@ YG_INLINE void emit_records(const Paths& P, const Queues& q, uint32_t slot, int 
         if (!(wt > 0.f) || !(wt < f_inf())) continue;
         if (pcg_float(rs, rinc) >= q.keep_prob) continue;
         // ring buffer over the whole render: training sees every pass's records, newest kept
-        const uint32_t idx = atomicAdd(&q.counts[10], 1u) % q.train_cap;
+        const uint32_t idx = atomicAdd(&q.counts[counter(10)], 1u) % q.train_cap;
         GuideRecord g;
         for (int j = 0; j < 9; j++) g.x[j] = R[j];
         g.wt = wt;
@@ -762,8 +800,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
     const Chunk& c = *cp;
     const uint32_t* in = parity ? q.active1 : q.active0;
     uint32_t* out = q.bin_rays ? q.unsorted : (parity ? q.active0 : q.active1);
-    uint32_t* n_out = &q.counts[parity ^ 1];
-    const uint32_t n = q.counts[parity];
+    uint32_t* n_out = &q.counts[counter(parity ^ 1)];
+    const uint32_t n = q.counts[counter(parity)];
     // The block takes its entries a window at a time and orders them by what they hit, so a wave shades one
     // kind of surface (or none) instead of every kind its lanes met.  Windows of 1,024 entries when they keep
     // the grid busy, else one round of the block.  (Lanes in use per issued vector instruction 0.40 to 0.66,
@@ -1351,8 +1389,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
             const uint64_t m = __ballot(mis_culled);
             if (__lane_id() == 0 && m) atomicAdd(&q.totals[20], (unsigned long long)__popcll(m));
         }
-        uint32_t* const light = q.counts + light_count_base(parity);
-        uint32_t* const ctr[4] = {n_out, &light[0], &light[1], &light[2]};
+        uint32_t* const light = q.counts + counter(light_count_base(parity));
+        uint32_t* const ctr[4] = {n_out, &light[counter(0)], &light[counter(1)], &light[counter(2)]};
         const bool pred[4] = {next_slot != kNoSlot, want_shadow, want_mis, want_dl};
         uint32_t qi[4];
         block_append<4>(ctr, pred, qi);
@@ -1375,7 +1413,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
             q.dl_shadow[id] = want_shadow ? is : kNoSlot;
         }
         if (GUIDED && c.guided) {
-            uint32_t* const gctr[1] = {&q.counts[9]};
+            uint32_t* const gctr[1] = {&q.counts[counter(9)]};
             const bool gpred[1] = {want_guide};
             uint32_t gidx[1];
             block_append<1>(gctr, gpred, gidx);
@@ -1402,8 +1440,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
 __global__ void k_guide_sample(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity) {
     const Chunk c = *cp;
     uint32_t* out = q.bin_rays ? q.unsorted : (parity ? q.active0 : q.active1);
-    uint32_t* n_out = &q.counts[parity ^ 1];
-    const uint32_t n = q.counts[9];
+    uint32_t* n_out = &q.counts[counter(parity ^ 1)];
+    const uint32_t n = q.counts[counter(9)];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t blk = blockIdx.x * blockDim.x; blk < n; blk += stride) {
         const uint32_t i = blk + threadIdx.x;
@@ -1478,7 +1516,7 @@ __global__ void k_guide_sample(DevScene s, const Chunk* __restrict__ cp, Paths P
 
 // Resolve, for the vertices the iteration before shaded: L += coeff * N * (light half + BSDF half) (path_tracing.cpp:56-57, direct_lighting.cpp:551)
 __global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Queues q, int parity) {
-    const uint32_t n = q.counts[light_count_base(parity ^ 1) + 2];
+    const uint32_t n = q.counts[counter(light_count_base(parity ^ 1) + 2)];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const uint32_t entry = q.dl_path[i], slot = entry & ~kDlMis, shadow = q.dl_shadow[i];
@@ -1505,7 +1543,7 @@ __global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Que
             if (c.deep == 2) {
                 const uint32_t next = take_parked(c, P, (int)pk.x, (int)pk.y + 1);
                 uint32_t* out = q.bin_rays ? q.unsorted : (parity ? q.active0 : q.active1);     // as k_shade appends
-                if (next != kNoSlot) out[atomicAdd(&q.counts[parity ^ 1], 1u)] = next;
+                if (next != kNoSlot) out[atomicAdd(&q.counts[counter(parity ^ 1)], 1u)] = next;
             }
         } else {
             P.L[slot] = f4(L, 0.f);
@@ -1515,11 +1553,11 @@ __global__ void k_resolve(DevScene s, const Chunk* __restrict__ cp, Paths P, Que
 }
 
 // Resets the counters an iteration appends to (a kernel, not a memset, so it can sit in a graph).
-__global__ void k_iter_reset(uint32_t* counts, int parity) {
+__global__ void k_iter_reset(uint32_t* counts, int parity, int cursors_end) {
     const int t = threadIdx.x;
-    if (t == 0) counts[parity ^ 1] = 0u;
-    else if (t <= 3) counts[light_count_base(parity) + t - 1] = 0u;
-    else if (t >= 6 && t <= 9) counts[t] = 0u;
+    if (t == 0) counts[counter(parity ^ 1)] = 0u;
+    else if (t <= 3) counts[counter(light_count_base(parity) + t - 1)] = 0u;
+    else if (t == 9 || (t >= kCounters && t < cursors_end)) counts[counter(t)] = 0u;
 }
 
 // Cube-map cell of a direction: dominant axis and sign pick one of 6 faces, the other two
@@ -1550,7 +1588,7 @@ __global__ __launch_bounds__(256) void k_bin_local(Paths P, Queues q, int parity
     __shared__ uint16_t s_key[kBinWindow];
     __shared__ uint32_t s_cur[NB];
     uint32_t* out = parity ? q.active0 : q.active1;
-    const uint32_t n = q.counts[parity ^ 1];
+    const uint32_t n = q.counts[counter(parity ^ 1)];
     const int t = threadIdx.x;
     for (uint32_t base = blockIdx.x * (uint32_t)kBinWindow; base < n; base += gridDim.x * (uint32_t)kBinWindow) {
         const int m = (int)min((uint32_t)kBinWindow, n - base);
@@ -1628,7 +1666,8 @@ int traversal_blocks_per_cu(const LaunchCfg& cfg) {
 void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p, Queues q, int parity, bool first, const LaunchCfg& cfg) {
     switch (stage) {
     case kStageReset:
-        hipLaunchKernelGGL(k_iter_reset, dim3(1), dim3(64), 0, cfg.stream, q.counts, parity);
+        hipLaunchKernelGGL(k_iter_reset, dim3(1), dim3(64), 0, cfg.stream, q.counts, parity,
+                           kCounters + kSlices * (cfg.split_kinds ? 3 : 1));
         break;
     case kStageBin:
         if (q.bin_rays == 1) hipLaunchKernelGGL(k_bin_local<2>, dim3(cfg.path_grid), dim3(256), 0, cfg.stream, p, q, parity);
@@ -1647,7 +1686,7 @@ void launch_stage(int stage, const DevScene& sc, const Chunk* c, const Paths& p,
 #undef YG_SHADE
         break;
     case kStageGuideForward:
-        if (cfg.guided) guide_forward_dev(cfg.net, q.guide_in, 16, &q.counts[9], q.guide_out, kGOut, cfg.guide_grid, cfg.stream);
+        if (cfg.guided) guide_forward_dev(cfg.net, q.guide_in, 16, &q.counts[counter(9)], q.guide_out, kGOut, cfg.guide_grid, cfg.stream);
         break;
     case kStageGuideSample:
         if (cfg.guided)
@@ -1749,7 +1788,7 @@ __global__ void k_film_spill(const Chunk* __restrict__ cp, Paths P, FilmParams f
                 }
             }
         if (margin) {
-            const uint32_t e = atomicAdd(&q.counts[5], 1u);
+            const uint32_t e = atomicAdd(&q.counts[counter(5)], 1u);
             if ((int)e < f.side_capacity) {
                 f.side_rad[e] = P.radiance[c.pix_first[p] + k];
                 f.side_info[e] = make_int4(px.x, px.y, k, (fp.x0 - px.x + 1) | ((fp.x1 - px.x) << 2) |
@@ -1856,39 +1895,66 @@ void launch_film(const Chunk* c, int n_pixels, const Paths& p, FilmParams f, Que
 }
 
 // ---------------------------------------------------------------------------------------------
-// Scene-tree ray queries for yar_gpu_trace_rays (32-byte yar_ray in, t/b + object/triangle out)
+// Scene-tree ray queries for yar_gpu_trace_rays (32-byte yar_ray in, 24-byte yar_hit out), by persistent
+// waves like the renderer's: lanes take new rays while others of their wave finish theirs, and a short
+// batch is spread over all waves (2^20 occlusion rays of the 2.2M-triangle scene: 468 us a call with
+// one ray per lane and a second kernel packing the hits, 456 us so).
 // ---------------------------------------------------------------------------------------------
 template <bool COUNT, bool PRIV>
-__global__ void k_trace_rays(DevScene sc, const float4* __restrict__ rays, long long n, int any, float4* out_tb,
-                             int2* out_ot, unsigned long long* totals, StackCfg cfg) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void YG_TRAV_BOUNDS k_trace_rays(DevScene sc, const float4* __restrict__ rays, uint32_t n, int any_hit, yar_hit* hits,
+                                            uint32_t* cursor, unsigned long long* totals, StackCfg cfg) {
     TravCounters cnt = {0, 0, 0, 0};
-    if (i < n) {
-        const float4 o4 = rays[2 * i], d4 = rays[2 * i + 1];
-        HitRec h;
-        with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
-            const bool found = trace<COUNT>(sc, from4(o4), from4(d4), o4.w, any != 0, h, st, depth, cnt);
-            if (any) {
-                out_tb[i] = make_float4(found ? 1.f : 0.f, 0.f, 0.f, 0.f);
-                out_ot[i] = make_int2(-1, -1);
-            } else if (found) {
-                const int tri_base = sc.obj_info[h.obj].w;
-                out_tb[i] = make_float4(h.t, h.b.x, h.b.y, h.b.z);
-                out_ot[i] = make_int2(h.obj, (int)h.tri - tri_base);
-            } else {
-                out_tb[i] = make_float4(f_inf(), 0.f, 0.f, 0.f);
-                out_ot[i] = make_int2(-1, -1);
-            }
-        });
-    }
+    with_stacks<PRIV>(cfg, [&](auto& st, int depth) {
+        trace_queue<COUNT>(sc, n, cursor, st, depth, cnt, cfg,
+            [&](uint32_t i, V3& o, V3& d, float& tmax, bool& any) -> uint32_t {
+                const float4 o4 = rays[2 * (size_t)i], d4 = rays[2 * (size_t)i + 1];
+                o = from4(o4);
+                d = from4(d4);
+                tmax = o4.w;
+                any = any_hit != 0;
+                return i;
+            },
+            [&](uint32_t i, const Tracer<COUNT>& tr) {
+                const bool closest = tr.result() && !tr.any;
+                yar_hit h;
+                h.t = tr.any ? (tr.result() ? 1.f : 0.f) : closest ? tr.hit.t : f_inf();
+                h.object = closest ? tr.hit.obj : -1;
+                h.triangle = closest ? (int)tr.hit.tri - sc.obj_info[tr.hit.obj].w : -1;
+                h.barycentrics[0] = closest ? tr.hit.b.x : 0.f;
+                h.barycentrics[1] = closest ? tr.hit.b.y : 0.f;
+                h.barycentrics[2] = closest ? tr.hit.b.z : 0.f;
+                hits[i] = h;
+            });
+    });
     flush_counters<COUNT>(totals, 3, cnt);
 }
 
-void launch_trace_rays(const DevScene& sc, const float4* rays, int64_t n, int any, float4* out_tb, int2* out_ot,
-                       unsigned long long* totals, const LaunchCfg& cfg) {
-    if (n <= 0) return;
-    const long long count = n;
-    YG_LAUNCH_TRAV(k_trace_rays, (count + cfg.block - 1) / cfg.block, sc, rays, count, any, out_tb, out_ot, totals);
+__global__ void k_clear_words(uint32_t* p, int n) {
+    if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
+}
+
+int trace_rays_blocks_per_cu(const LaunchCfg& cfg) {
+    int nb = 0;
+    const size_t shm = stack_lds(cfg);
+    const hipError_t e = cfg.priv_stack ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_trace_rays<false, true>), cfg.block, shm)
+                                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_trace_rays<false, false>), cfg.block, shm);
+    if (e != hipSuccess || nb <= 0) nb = 1;
+    return nb;
+}
+
+void launch_trace_rays(const DevScene& sc, const float4* rays, int64_t n, int any, yar_hit* hits, unsigned long long* totals,
+                       const LaunchCfg& cfg) {
+    // counters and cursors are only used by counted calls and where the waves' first runs do not cover the batch
+    const int64_t first_runs = (int64_t)cfg.trav_grid * (cfg.block / 64) * 64;
+    constexpr int64_t kMost = (int64_t)1 << 30;               // rays of one launch
+    uint32_t* words = reinterpret_cast<uint32_t*>(totals);
+    const bool clear = cfg.counters || n >= first_runs;
+    for (int64_t at = 0; at < n; at += kMost) {
+        const uint32_t m = (uint32_t)std::min(kMost, n - at);
+        const int from = at == 0 ? 0 : kCounterWords;         // later launches add to the counters
+        if (clear) hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(1024), 0, cfg.stream, words + from, kRayWords - from);
+        YG_LAUNCH_TRAV(k_trace_rays, cfg.trav_grid, sc, rays + 2 * at, m, any, hits + at, words + kCounterWords, totals);
+    }
 }
 
 }  // namespace yg
