@@ -939,8 +939,8 @@ static void render_job(yar_gpu_ctx* ctx, const std::vector<JobPart>& parts, std:
 
     // chunks of whole tiles, bounded by paths in flight, sample-table and radiance sizes.
     // Plain jobs default to 64M paths in flight: the persistent traversal kernels need wide queues in
-    // the late bounces, where most paths have ended (config 2, 1024x1024 at 64 spp: 262 Msamples/s at
-    // 4M paths, 329 at 8M, 390 at 16M, 416 at 32M in two chunks, 449 at 64M in one chunk).  Guided
+    // the late bounces, where most paths have ended (1024x1024 at 64 spp of the 2.2M-triangle scene: 723
+    // Msamples/s at 4M paths, 829 at 8M, 902 at 16M, 927 at 32M in two chunks, 980 at 64M in one chunk).  Guided
     // jobs revisit every chunk once per pass and keep up to 16M paths in one chunk.  Path state is
     // about 265 B per path (plain: 13 float4 rays / throughputs / direct-lighting halves / queue
     // payloads, hit, state and 5 queue slots; 64M paths hold about 19 GB) and about 800 B guided

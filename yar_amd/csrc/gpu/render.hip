@@ -550,7 +550,7 @@ YG_INLINE void with_stacks(StackCfg cfg, Body body) {
 // ticket of the run behind the current one is drawn when the current one is begun, so its 1 to 2 us pass
 // while the wave traces.  Within the last kAhead entries per wave no ticket is drawn ahead: a wave busy with
 // long rays would hold a run that idle waves could take.  (One cursor, fetched when needed:
-// seven 512x512 views of a small room in one batch 16.2 ms, 1024x1024 at 64 spp of the 2.2M-triangle scene
+// seven views of a small room, up to 512x512, in one batch 16.2 ms, 1024x1024 at 64 spp of the 2.2M-triangle scene
 // 67.7; so 14.6 and 65.5.  Eight cursors, looked at before each draw and none drawn early: 16.8 and 75.)
 // A lane whose query ended takes the run's next entry once cfg.refill lanes of its wave are idle, so a wave
 // is not held by its longest ray (24 idle lanes against 64, i.e. whole batches: 84 against 103 ms on the
@@ -644,8 +644,7 @@ YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Sta
     }
 }
 
-// Registers capped for the five waves per SIMD that the stacks' LDS allows (80 to 90 VGPRs, no spills; a
-// sixth wave needs 80, spills 28 B in k_extend and gains nothing).  Blocks of at most 256 threads.
+// Registers capped for the five waves per SIMD that the stacks' LDS allows (92 VGPRs, no spills).  Blocks of at most 256 threads.
 #define YG_TRAV_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 
 // A BSDF-sampled light ray's contribution (direct_lighting.cpp:163-191 and its sphere, mesh and environment
