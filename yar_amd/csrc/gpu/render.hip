@@ -543,10 +543,10 @@ YG_INLINE void with_stacks(StackCfg cfg, Body body) {
 }
 
 // Persistent traversal over a device queue.  A queue of 64 entries per wave or more is cut into kSlices
-// slices, and the blocks of an XCD (dealt round-robin) start on one of them.  A wave takes runs of entries:
-// the first one is its by position, the others come from its slice's cursor, 256 entries at a time while
-// more than 8 such fetches per wave remain, then 64 (balanced tail), and from the other slices once its own
-// is done.  One cursor per slice, on a line of its own, because atomics on one address serialize; and the
+// slices, and the blocks of an XCD (dealt round-robin) start on one of them.  A wave takes runs of 64
+// entries: the first one is its by position, the others come from its slice's cursor, and from the other
+// slices once its own is done (runs of 256
+// entries until eight per wave are left: 14.7 against 14.5 ms on the batch below, 65.8 against 65.4 on the frame).  One cursor per slice, on a line of its own, because atomics on one address serialize; and the
 // ticket of the run behind the current one is drawn when the current one is begun, so its 1 to 2 us pass
 // while the wave traces.  Within the last kAhead entries per wave no ticket is drawn ahead: a wave busy with
 // long rays would hold a run that idle waves could take.  (One cursor, fetched when needed:
@@ -560,8 +560,7 @@ YG_INLINE void with_stacks(StackCfg cfg, Body body) {
 // 63 others (64x64 tile at 4 spp: 2.7 to 1.7 ms per render).  It is not cut into slices: path, shadow and MIS
 // rays would lie on XCDs of their own, of unequal length (0.92 to 0.96 ms per render).
 // setup(index, o, d, tmax, any) returns the payload finish(payload, tracer) receives.
-constexpr uint32_t kNoTicket = 0xffffffffu, kAhead = 6u * 64u;
-YG_INLINE bool long_runs(uint32_t n, uint32_t waves) { return n > 8u * 256u * waves; }
+constexpr uint32_t kNoTicket = 0xffffffffu, kRun = 64u, kAhead = 6u * kRun;
 template <bool COUNT, class Stack, class Setup, class Finish>
 YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Stack& st, int depth, TravCounters& cnt,
                            StackCfg cfg, Setup setup, Finish finish) {
@@ -570,50 +569,46 @@ YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Sta
     const uint32_t wpb = (blockDim.x + 63u) >> 6;
     const uint32_t lane = __lane_id();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool spread = n < 64u * gridDim.x * wpb;
-    uint32_t size, slice = 0u, slices_left = 0u, next, end;
+    uint32_t slice = 0u, slices_left = 0u, next, end;
     uint32_t ticket = kNoTicket;        // in lane 0
     // first entry of slice s's cursor, first entry behind the slice, and the entries one run per wave takes
-    auto bounds = [&](uint32_t n, uint32_t s, uint32_t run, uint32_t& base, uint32_t& stop, uint32_t& round) {
+    auto bounds = [&](uint32_t n, uint32_t s, uint32_t& base, uint32_t& stop, uint32_t& round) {
         const uint32_t part = (n + kSlices - 1u) / kSlices;
-        round = gridDim.x > s ? (gridDim.x - s + kSlices - 1u) / kSlices * wpb * run : 0u;
+        round = gridDim.x > s ? (gridDim.x - s + kSlices - 1u) / kSlices * wpb * kRun : 0u;
         stop = min((s + 1u) * part, n);
         base = min(s * part, n) + round;
     };
-    if (spread) {
-        size = max(1u, (n + gridDim.x * wpb - 1u) / (gridDim.x * wpb));
+    if (n < kRun * gridDim.x * wpb) {
+        const uint32_t size = max(1u, (n + gridDim.x * wpb - 1u) / (gridDim.x * wpb));
         next = min((blockIdx.x * wpb + wave) * size, n);
         end = min(next + size, n);
     } else {
-        size = long_runs(n, gridDim.x * wpb) ? 256u : 64u;
         slice = blockIdx.x % kSlices;
         slices_left = kSlices;
         uint32_t base, stop, round;
-        bounds(n, slice, size, base, stop, round);
-        next = min(base - round + (blockIdx.x / kSlices * wpb + wave) * size, stop);
-        end = min(next + size, stop);
-        if (base < stop && stop - base > kAhead / size * round && lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, size);
+        bounds(n, slice, base, stop, round);
+        next = min(base - round + (blockIdx.x / kSlices * wpb + wave) * kRun, stop);
+        end = min(next + kRun, stop);
+        if (base < stop && stop - base > kAhead / kRun * round && lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, kRun);
     }
     // the next run of the wave's slice, or of the first one behind it that is not used up
     auto fetch = [&]() {
         uint32_t m = n;
         asm volatile("" : "+s"(m));     // computed again here, not kept in registers the traversal needs
-        const uint32_t run = long_runs(m, gridDim.x * wpb) ? 256u : 64u;
         for (; slices_left > 0u; slices_left--, slice = (slice + 1u) % kSlices) {
             uint32_t base, stop, round;
-            bounds(m, slice, run, base, stop, round);
+            bounds(m, slice, base, stop, round);
             if (base >= stop) continue;
             uint32_t at = __builtin_amdgcn_readfirstlane(ticket);
             if (at == kNoTicket) {
-                if (lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, size);
+                if (lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, kRun);
                 at = __builtin_amdgcn_readfirstlane(ticket);
             }
             ticket = kNoTicket;
             if (at >= stop - base) continue;
             next = base + at;
-            end = min(next + size, stop);
-            if (size > 64u && !long_runs((stop - end) * kSlices, gridDim.x * wpb)) size = 64u;
-            if (stop - end > kAhead / run * round && lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, size);
+            end = min(next + kRun, stop);
+            if (stop - end > kAhead / kRun * round && lane == 0) ticket = atomicAdd(cursor + slice * kCounterWords, kRun);
             return;
         }
     };
@@ -644,7 +639,7 @@ YG_INLINE void trace_queue(const DevScene& sc, uint32_t n, uint32_t* cursor, Sta
     }
 }
 
-// Registers capped for the five waves per SIMD that the stacks' LDS allows (92 VGPRs, no spills).  Blocks of at most 256 threads.
+// Registers capped for the five waves per SIMD that the stacks' LDS allows (93 VGPRs, no spills).  Blocks of at most 256 threads.
 #define YG_TRAV_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 
 // A BSDF-sampled light ray's contribution (direct_lighting.cpp:163-191 and its sphere, mesh and environment
