@@ -545,13 +545,13 @@ YG_INLINE void with_stacks(StackCfg cfg, Body body) {
 // Persistent traversal over a device queue.  A queue of 64 entries per wave or more is cut into kSlices
 // slices, and the blocks of an XCD (dealt round-robin) start on one of them.  A wave takes runs of 64
 // entries: the first one is its by position, the others come from its slice's cursor, and from the other
-// slices once its own is done (runs of 256
-// entries until eight per wave are left: 14.7 against 14.5 ms on the batch below, 65.8 against 65.4 on the frame).  One cursor per slice, on a line of its own, because atomics on one address serialize; and the
-// ticket of the run behind the current one is drawn when the current one is begun, so its 1 to 2 us pass
-// while the wave traces.  Within the last kAhead entries per wave no ticket is drawn ahead: a wave busy with
-// long rays would hold a run that idle waves could take.  (One cursor, fetched when needed:
-// seven views of a small room, up to 512x512, in one batch 16.2 ms, 1024x1024 at 64 spp of the 2.2M-triangle scene
-// 67.7; so 14.6 and 65.5.  Eight cursors, looked at before each draw and none drawn early: 16.8 and 75.)
+// slices once its own is done.  One cursor per slice, on a line of its own, because atomics on one address
+// serialize; and the ticket of the run behind the current one is drawn when the current one is begun, so
+// its 1 to 2 us pass while the wave traces.  Within the last kAhead entries per wave no ticket is drawn
+// ahead: a wave busy with long rays would hold a run that idle waves could take.  (One cursor, fetched when
+// needed: seven views of a small room, up to 512x512, in one batch 16.2 ms, 1024x1024 at 64 spp of the
+// 2.2M-triangle scene 67.7; so 14.5 and 65.4; with runs of 256 entries until eight per wave are left 14.7
+// and 65.8; eight cursors, looked at before each draw and none drawn early, 16.8 and 75.)
 // A lane whose query ended takes the run's next entry once cfg.refill lanes of its wave are idle, so a wave
 // is not held by its longest ray (24 idle lanes against 64, i.e. whole batches: 84 against 103 ms on the
 // 1024x1024 frame of the 2.2M-triangle scene, 8 and 32 within 1%).
